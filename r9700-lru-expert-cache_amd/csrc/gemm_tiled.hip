@@ -6,7 +6,7 @@
 //                  at most TMB blocks; a tile is (first block, block count). Blocks of expert -1
 //                  make no tile. Given two aligns (a layer's resident and non-resident rows),
 //                  it lists the second one's tiles after the first one's, with bit 16 of the
-//                  block count set; only the streamed kernel (prefill.hip) reads such a list.
+//                  block count set; only the streamed kernels (prefill.h) read such a list.
 //   tiled_k        one workgroup (8 waves) computes a TMB*16-row x 256-column tile: per 128-deep
 //                  K step it stages the tile's activation rows (gathered through sorted_ids) and
 //                  the 16 weight strips (fragment order, 2 KB contiguous each) in LDS, double-
@@ -295,7 +295,7 @@ static int check_gemm_args(int mtk, int top_k, int K, int N, int max_tiles, int 
   return 0;
 }
 
-// The streamed kernel (prefill.hip) where K and N have a built configuration, tiled_k
+// A streamed kernel (prefill.hip, prefill_roll.hip) where one takes K and N, tiled_k
 // otherwise; both give the same bits.
 static void launch_tiled(const void* qx, const float* xs, const void* wq, const float* ws,
                          const int* sorted_ids, const int* expert_ids, const int* tiles,
@@ -376,7 +376,7 @@ int rlu_moe_gemm_fp8blk_tiled_noalloc(const void* qx, const float* xs, const voi
   return (int)hipGetLastError();
 }
 
-// The gate_up GEMM with SiLU-mul-quant fused into its epilogue (prefill.hip, ACT): q2 / s2
+// The gate_up GEMM with SiLU-mul-quant fused into its epilogue (prefill_roll.hip): q2 / s2
 // equal rlu_silu_mul_quant (group 128) of rlu_moe_gemm_fp8blk_tiled's bf16 output bit for bit,
 // without that [mtk, N] output. Built for K = 2560 (gate_up of the 2560-wide model) and N % 256
 // == 0; other shapes return -6 before anything else is checked, so a call with mtk = 0 is a

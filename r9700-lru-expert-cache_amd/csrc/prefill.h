@@ -1,5 +1,5 @@
-// The streamed prefill grouped GEMM (prefill.hip), launched by the tiled entry points of
-// gemm_tiled.hip for the K it is built for.
+// The streamed prefill grouped GEMMs (prefill.hip, prefill_roll.hip), launched by the tiled entry
+// points of gemm_tiled.hip for the K they take.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -14,12 +14,12 @@ struct PfSecond {
   const int* expert_ids;
 };
 
-// K and N with a built configuration of the plain streamed kernel.
+// K and N of the two-set launches.
 bool prefill_stream_built(int K, int N);
 
-// Launches the streamed kernel over a tile list (tiles of <= 8 blocks) when K and N have a
-// built configuration, and returns 0; returns -1 (nothing launched) otherwise. second: null
-// for a one-set tile list.
+// Launches a streamed kernel over a tile list (tiles of <= 8 blocks) when one takes K and N (K =
+// 768 or a multiple of 512 from 1024 on, N % 256 == 0), and returns 0; returns -1 (nothing
+// launched) otherwise. second: null for a one-set tile list.
 int launch_prefill_stream(const void* qx, const float* xs, const void* wq, const float* ws,
                           const int* sorted_ids, const int* expert_ids, const PfSecond* second,
                           const int* tiles, const int* ntiles, int max_tiles,

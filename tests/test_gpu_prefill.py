@@ -1,0 +1,130 @@
+"""The streamed prefill GEMMs (the unrolled K = 768 kernel and the rolled one for K a multiple of 512
+from 1024 on) against the general tiled kernel, which runs the same sequence of operations per
+output: equal bit for bit, over row distributions that take each branch of the tiles' schedule.
+"""
+from __future__ import annotations
+
+import pytest
+
+from conftest import gpu_case
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def ops(pkg):
+    from importlib import import_module
+    return import_module(pkg.__name__ + ".ops")
+
+
+# rows per expert: tiles of one and of several per expert mixed, at 24 rows per tile or more (the
+# workgroups are split between the two kinds) and below (list order); only one kind; fewer items
+# than XCDs; no tile at all.
+ROWS = {
+    "mixed": [300, 5, 40, 17, 128, 129, 1, 0, 16, 700, 96, 250, 33] * 4,
+    "mixed_few": [300, 40, 130],
+    "alone": [128, 100, 90, 77] * 6,
+    "shared": [400] * 5,
+    "thin": [9] * 40 + [200],
+    "one": [3],
+    "none": [],
+}
+SHAPES = [(768, 512), (1024, 256), (1536, 256), (2048, 768), (2560, 512), (4096, 256)]
+
+
+def align(rows, order):
+    """One align of mtk = sum(rows) ids dealt to the experts in the given order."""
+    mtk = sum(rows)
+    sid, eid, pos = [], [], 0
+    for e, r in enumerate(rows):
+        nb = (r + 15) // 16
+        sid += order[pos:pos + r] + [mtk] * (nb * 16 - r)
+        eid += [e] * nb
+        pos += r
+    dev = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    n = len(eid)
+    return dev(sid or [mtk] * 16), dev(eid or [-1]), dev([16 * n])
+
+
+def weights(E, N, K, gen):
+    """Finite e4m3 bytes (0x7f and 0xff are NaN) and positive block scales."""
+    w = torch.randint(0, 256, (E, N, K), dtype=torch.uint8, generator=gen, device=DEV)
+    w = torch.where((w & 0x7f) == 0x7f, w ^ 1, w).view(torch.float8_e4m3fn)
+    return w, torch.rand(E, N // 128, K // 128, generator=gen, device=DEV) * 0.01
+
+
+def tile_list(rows):
+    """moe_gemm_tiles of that align, where it has more blocks than the builder takes."""
+    out, b = [], 0
+    for r in rows:
+        nb = (r + 15) // 16
+        for s in range(0, nb, 8):
+            out += [b + s, min(8, nb - s)]
+        b += nb
+    out = out + [0] * (2 * b - len(out)) + [len(out) // 2]
+    return torch.tensor(out, dtype=torch.int32, device=DEV)
+
+
+def check(ops, name, rows, K, N, routed, E=None):
+    gen = torch.Generator(DEV).manual_seed(K + N)
+    E = E or max(len(rows), 1)
+    mtk = max(sum(rows), 1)
+    w, ws = weights(E, N, K, gen)
+    order = torch.randperm(mtk, generator=torch.Generator().manual_seed(1)).tolist()
+    al = align(rows, order)
+    if len(rows) > E:
+        al[1].remainder_(E)                          # neighbours stay of different experts
+    tiles = tile_list(rows) if len(rows) > E else None
+    qx = torch.randint(0, 0x7f, (mtk, K), dtype=torch.uint8, generator=gen, device=DEV)
+    qx = (qx ^ 0x80 * (qx & 1)).view(torch.float8_e4m3fn)     # signs by the lowest bit
+    xs = torch.rand(mtk, K // 128, generator=gen, device=DEV)
+    tw = torch.rand(mtk, generator=gen, device=DEV) if routed else None
+    out = []
+    for wv in (0, 2):
+        y = torch.full((mtk, N), 7.0, dtype=torch.bfloat16, device=DEV)
+        gpu_case(f"streamed prefill gemm {name} K={K} N={N} wv={wv}")
+        ops.moe_gemm_tiled(y, qx, xs, w, ws, *al, tw, mtk, 1, wv=wv, tiles=tiles,
+                           tiles_ready=tiles is not None)
+        torch.cuda.synchronize()
+        out.append(y.view(torch.int16))
+    assert torch.equal(*out)
+    assert bool((out[0] != 0x40e0).any()) == bool(rows)      # 7.0 where nothing was written
+
+
+@pytest.mark.parametrize("K,N", SHAPES)
+@pytest.mark.parametrize("name", ROWS)
+def test_streamed_equals_general_tiled(ops, name, K, N):
+    check(ops, name, ROWS[name], K, N, routed=N % 512 == 0)
+
+
+@pytest.mark.parametrize("K", [768, 1024])
+@pytest.mark.parametrize("n", [16000, 16380, 17000])
+def test_streamed_at_the_orders_capacity(ops, n, K):
+    """Tiles up to what the XCDs' orders hold (2048 each), and past that and past what the
+    scheduler takes (16384)."""
+    check(ops, f"{n} tiles", [40] * n + [200], K, 256, routed=True, E=64)
+
+
+def test_streamed_activations_past_2gb(ops):
+    """Row offsets past 31 bits take the 64-bit addresses: 2.2 GB of activations, of which the
+    align names rows at both ends."""
+    tokens, K, N = 860_000, 2560, 256
+    gen = torch.Generator(DEV).manual_seed(7)
+    w, ws = weights(3, N, K, gen)
+    qx = torch.randint(0, 0x7f, (tokens, K), dtype=torch.uint8, generator=gen,
+                       device=DEV).view(torch.float8_e4m3fn)
+    xs = torch.rand(tokens, K // 128, generator=gen, device=DEV)
+    ids = list(range(300)) + list(range(tokens - 212, tokens))
+    sid = torch.tensor(ids, dtype=torch.int32, device=DEV)
+    eid = torch.tensor([0] * 10 + [1] * 3 + [2] * 19, dtype=torch.int32, device=DEV)
+    npad = torch.tensor([512], dtype=torch.int32, device=DEV)
+    out = []
+    for wv in (0, 2):
+        y = torch.zeros(tokens, N, dtype=torch.bfloat16, device=DEV)
+        gpu_case(f"streamed prefill gemm, activations past 2 GB, wv={wv}")
+        ops.moe_gemm_tiled(y, qx, xs, w, ws, sid, eid, npad, None, tokens, 1, wv=wv)
+        torch.cuda.synchronize()
+        out.append(y.view(torch.int16))
+    assert torch.equal(*out) and bool(out[0][ids].any())
