@@ -181,6 +181,12 @@ int rlu_moe_gemm_split_qin(const void* act, const void* wq_hot, const float* ws_
 int rlu_gemm_fp8blk_m16(const void* qx, const float* xs, const void* w, const float* ws,
                         void* y, int M, int N, int K, int wv, int npw, hipStream_t stream);
 
+/* The same for 1 <= M <= 64 with the weights read once for all rows; every row equals
+ * rlu_gemm_fp8blk_m16's bit for bit. Returns -1 (bad sizes or a NULL pointer), -2 (K % 128 or N %
+ * 128), -4 (K / 128 over its split too long, as rlu_gemm_fp8blk_m16). */
+int rlu_gemm_fp8blk_m64(const void* qx, const float* xs, const void* w, const float* ws,
+                        void* y, int M, int N, int K, hipStream_t stream);
+
 /* Replaces shuffle_weight_gfx1201 (the load-time weight shuffle behind pack_fp8_block,
  * kernels/fp8_target_lmhead.py:44-66) for gfx950: row-major e4m3 [rows, K] -> MFMA fragment
  * order, the layout every GEMM above reads. Byte (n, k), n = 16 nt + r,
