@@ -320,6 +320,11 @@ int rlu_moe_gemm_fp8blk_tiled_noalloc(const void* qx, const float* xs, const voi
 int rlu_gemm_w4_m16(const void* x, int M, int K, const void* wq, const unsigned* sz, void* y,
                     int N, int wv, hipStream_t stream);
 
+/* The same for 17 <= M <= 64 in one read of the weight, to within the rounding of f32 sums taken in
+ * another order. Returns as rlu_gemm_w4_m16. */
+int rlu_gemm_w4_m64(const void* x, int M, int K, const void* wq, const unsigned* sz, void* y,
+                    int N, hipStream_t stream);
+
 /* Replaces quantize_w4 + pack_w4a16 (kernels/draft_w4_lmhead.py:154-198,228-259), with this
  * build's own quantizer, in the format rlu_gemm_w4_m16 reads: w [N, K] (row stride ld elements,
  * 16-byte aligned rows; dtype 0 bf16, 1 f32, 2 f16) -> wq [n_pad/16][K/128][64][16] codes and

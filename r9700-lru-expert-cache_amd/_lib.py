@@ -37,6 +37,7 @@ SIGNATURES: dict[str, tuple] = {
     "rlu_shuffle_fp8_weight": (_I, [_P, _P, _LL, _I, _P]),
     "rlu_gemm_fp8blk_m64": (_I, [_P] * 5 + [_I] * 3 + [_P]),
     "rlu_gemm_w4_m16": (_I, [_P, _I, _I, _P, _P, _P, _I, _I, _P]),
+    "rlu_gemm_w4_m64": (_I, [_P, _I, _I, _P, _P, _P, _I, _P]),
     "rlu_pack_w4": (_I, [_P, _I, _LL, _I, _I, _I, _P, _P, _P]),
     "rlu_moe_gemm_tiles": (_I, [_P, _P, _I, _P, _P, _P]),
     "rlu_moe_gemm_fp8blk_tiled": (_I, [_P] * 8 + [_I, _P, _P] + [_I] * 5 + [_P]),

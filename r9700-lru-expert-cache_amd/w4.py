@@ -19,7 +19,8 @@ the group's range (bf16 scale) and, for each, the centred integer zero and its t
 and keeps the least squared error; a constant group is stored exactly up to the bf16 scale.
 The reference stores an f16 scale and widens bf16 activations to f16 for its gfx1201 WMMA; here
 the activations stay bf16. N is padded to a multiple of 32 (the GEMV's item is two 16-row
-strips) with zero rows, sliced off again by the op. M > 16 runs the kernel on 16-row slices.
+strips) with zero rows, sliced off again by the op. M > 16 reads the weight once per
+64 rows (rlu_gemm_w4_m64).
 """
 from __future__ import annotations
 
@@ -137,18 +138,26 @@ def _gemm_into(x: torch.Tensor, packed_wq: torch.Tensor, packed_sz: torch.Tensor
                y: torch.Tensor, wv: int) -> None:
     m = x.shape[0]
     n_pad = packed_wq.shape[0] * 16
-    for r0 in range(0, m, MAX_M):
-        r1 = min(m, r0 + MAX_M)
-        rc = lib().rlu_gemm_w4_m16(_P(x[r0:r1].data_ptr()), r1 - r0, k,
-                                   _P(packed_wq.data_ptr()), _P(packed_sz.data_ptr()),
-                                   _P(y[r0:r1].data_ptr()), n_pad, wv, _P(stream_ptr()))
-        check(rc, "rlu_gemm_w4_m16")
+    r0 = 0
+    while r0 < m:
+        # up to 64 rows share one read of the weight; a rest of at most 16, or a given wv, runs the
+        # 16-row kernel (16 rows at vocab 151936 x 2560: 42-46 us on either, 32000 x 4096: 23 and
+        # 24, 4096 x 2560: 13 and 17; 17 rows: 85 and 49, 42 and 29, 20 and 20)
+        many = m - r0 > MAX_M and not wv
+        r1 = min(m, r0 + (4 * MAX_M if many else MAX_M))
+        a = (_P(x[r0:r1].data_ptr()), r1 - r0, k, _P(packed_wq.data_ptr()),
+             _P(packed_sz.data_ptr()), _P(y[r0:r1].data_ptr()), n_pad)
+        if many:
+            check(lib().rlu_gemm_w4_m64(*a, _P(stream_ptr())), "rlu_gemm_w4_m64")
+        else:
+            check(lib().rlu_gemm_w4_m16(*a, wv, _P(stream_ptr())), "rlu_gemm_w4_m16")
+        r0 = r1
 
 
 def _draft_w4_lmhead_gemm(x: torch.Tensor, wq: torch.Tensor, wsz: torch.Tensor, n: int,
                           k: int, wv: int, sk: int, npw: int, nt: int) -> torch.Tensor:
     """The op of kernels/draft_w4_lmhead.py:351-390: [M, K] hidden states -> [M, n] bf16
-    logits, every M in one opaque call (16-row slices inside). wv = workgroups per CU of the
+    logits, every M in one opaque call (64- and 16-row slices inside). wv = workgroups per CU of the
     kernel's persistent grid (0: the kernel's default). sk / npw / nt name the closed kernel's
     K split, columns per wave and tile shape; this kernel derives its K split from K and has one
     item shape, so they are accepted for the schema (non-negative) and not used."""
