@@ -207,7 +207,8 @@ int rlu_moe_gemm_tiles(const int* expert_ids, const int* num_post_pad, int nb_ma
  * r4d_gemm_moe_fp8blk_nt_b16 with sk = 1 (equal to it bit for bit), one workgroup per 128-row x
  * 256-column tile so an expert's weights are read once per tile. max_tiles bounds the device
  * count (the align output's block count). N % 256 == 0. wv = 0 picks a streamed kernel where
- * one takes K (768, or a multiple of 512 from 1024 on; persistent, one workgroup per CU walking
+ * one takes the shape (K = 768, a multiple of 512 from 1024 on, or any K from 512 on when the rows
+ * make two items per CU; persistent, one workgroup per CU walking
  * (tile, 256-column strip) items with the weight stream kept in flight across items), else the
  * general tiled kernel at 2 workgroups per CU; wv in
  * 1..16 forces the general kernel at wv workgroups per CU. Every choice gives the same bits.

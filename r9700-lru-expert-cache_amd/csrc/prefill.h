@@ -18,7 +18,7 @@ struct PfSecond {
 bool prefill_stream_built(int K, int N);
 
 // Launches a streamed kernel over a tile list (tiles of <= 8 blocks) when one takes K and N (K =
-// 768 or a multiple of 512 from 1024 on, N % 256 == 0), and returns 0; returns -1 (nothing
+// 768, or what roll_takes says, N % 256 == 0), and returns 0; returns -1 (nothing
 // launched) otherwise. second: null for a one-set tile list.
 int launch_prefill_stream(const void* qx, const float* xs, const void* wq, const float* ws,
                           const int* sorted_ids, const int* expert_ids, const PfSecond* second,

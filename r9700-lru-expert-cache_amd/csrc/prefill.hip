@@ -1,7 +1,7 @@
 // The grouped fp8 GEMM of a prefill chunk (tens of rows per expert), streamed: same operands,
 // row contract, tile list and numerics as tiled_k (gemm_tiled.hip) and moe_gemm_k (gemm.hip),
-// bit for bit, for K = 768 (down of the 2560-wide model). A K that is a multiple of 512 from 1024
-// on runs the rolled form (prefill_roll.hip), any other K tiled_k.
+// bit for bit, for K = 768 (down of the 2560-wide model). Other K run the rolled form
+// (prefill_roll.hip, roll_takes) or tiled_k.
 //
 // The unrolled form stays here because an item of 6 steps is short: the ring holds a whole item
 // ahead, and the rolled form's per-chunk work costs 5% at one block per tile (193 against 203 us).
@@ -395,6 +395,18 @@ static pf::Args make_args(const void* qx, const float* xs, const void* wq, const
 
 bool prefill_stream_built(int K, int N) { return (K == 2560 || K == 768) && N % 256 == 0; }
 
+// The rolled kernel's K: a multiple of its chunk of 4 steps from two chunks on; any other K from one
+// chunk on once the rows alone make two items per CU (64 experts, 8192 tokens, down of K = 1408
+// 533 -> 401 us, 2048 tokens 152 -> 149; 32 experts, 2048 tokens, K = 896 103 -> 86). Below, its one
+// workgroup per CU leaves a part of the CUs idle in the last round, and a short or broken K makes
+// up for less of that (32 experts, 512 tokens, K = 896: 52 against 46 us of tiled_k; 256 experts, 64
+// tokens, K = 512: 45 against 39).
+static bool roll_takes(int mtk, int K, int N) {
+  if (K % 128 || K < 512) return false;
+  return (K % 512 == 0 && K >= 1024) ||
+         (long long)mtk * N >= 2LL * 16 * pf::TB * 256 * device_cus();
+}
+
 int launch_prefill_stream(const void* qx, const float* xs, const void* wq, const float* ws,
                           const int* sorted_ids, const int* expert_ids, const PfSecond* second,
                           const int* tiles, const int* ntiles, int max_tiles,
@@ -405,7 +417,7 @@ int launch_prefill_stream(const void* qx, const float* xs, const void* wq, const
                                topk_weights, y, nullptr, nullptr, mtk, top_k, K, N);
   if (K == 768)
     pf::launch_k768(a, max_tiles, stream);
-  else if (K % 512 == 0 && K >= 1024)
+  else if (roll_takes(mtk, K, N))
     pf::launch_roll(a, max_tiles, stream);
   else
     return -1;

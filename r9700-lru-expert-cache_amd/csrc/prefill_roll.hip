@@ -1,5 +1,5 @@
 // The rolled prefill GEMM: same items, operands, tile list and numerics as the unrolled kernel of
-// prefill.hip (equal bit for bit), for K a run-time multiple of 512 from 1024 on, with the K loop a
+// prefill.hip (equal bit for bit), for K a run-time multiple of 128 from 512 on, with the K loop a
 // loop and each step software-pipelined. It runs gate_up of the 2560-wide model, alone or
 // with SiLU-mul-quant in its epilogue, and both GEMMs of shapes with such a K: at 2048 / 8192
 // tokens over 128 experts gate_up (K 2048, N 1536) takes 143 / 400 us, tiled_k 190 / 565; over 64
@@ -71,7 +71,7 @@ __device__ __forceinline__ float quad(float x) {
 // exactly as silu_mul_quant_k computes them from y (same silu, product and amax reduction, same
 // rounding). TWT: routed weights. TWO: the tile list covers two aligns (bit 16 of a tile's block
 // count picks the set). POL: the weight loads' cache policy.
-template <int POL, bool TWT, bool ACT, bool TWO, bool WIDE>
+template <int POL, bool TWT, bool ACT, bool TWO, bool WIDE, bool TAIL>
 __device__ __forceinline__ void items(
     const Sched& sc, const uint8_t* __restrict__ qx, const float* __restrict__ xs,
     const uint8_t* __restrict__ wq, const float* __restrict__ ws,
@@ -91,7 +91,10 @@ __device__ __forceinline__ void items(
   const int w = uniform((int)(threadIdx.x / WAVE));
   const int r16 = lane & 15, c4 = lane >> 4;
   const int cb = w / (NWAVE / 2);                       // this wave's 128-column scale block
-  const int nk = K / 128, nch = nk / KC;
+  const int nk = K / 128;
+  // TAIL: the last chunk has what KC leaves of K / 128, nothing where that is one chunk alone (the
+  // metadata pipeline takes two)
+  const int nch = TAIL ? max(2, (nk + KC - 1) / KC) : nk / KC;
   const int ncg = N / C;
   // first output column of scale block h of an item starting at column n0
   auto bcol = [&](int n0, int h) __attribute__((always_inline)) -> int {
@@ -132,10 +135,12 @@ __device__ __forceinline__ void items(
   };
   // this wave's strips of an item, as a buffer: strip s, step k, half h at s 16 K + k 2048 +
   // h 1024 + lane 16 (the base and the step offset stay in scalar registers)
-  auto wbase = [&](const Item& it) __attribute__((always_inline)) {
-    return __builtin_amdgcn_make_buffer_rsrc(
-        (void*)((it.set ? wq1 : wq) + ((size_t)it.e * N + bcol(it.n0, cb) + wcol) * K), 0,
-        S * 16 * K, BUF_WORD3);
+  // steps: 0 for a buffer whose loads touch no memory
+  auto wbuf = [&](const uint8_t* p, bool any) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, any ? S * 16 * K : 0, BUF_WORD3);
+  };
+  auto wptr = [&](const Item& it) __attribute__((always_inline)) {
+    return (it.set ? wq1 : wq) + ((size_t)it.e * N + bcol(it.n0, cb) + wcol) * K;
   };
 
   // ---- registers ----
@@ -158,7 +163,7 @@ __device__ __forceinline__ void items(
   // the activation rows and their scales, and the item's weight scales
   struct Rows {
     int va;                           // byte offset of the row, + 16 c4 (WIDE: the row)
-    int vx;                           // index of the row's scales, + this lane's step
+    int vx;                           // index of the row's scales
     const float* w0;                  // weight scales of the first column block (scalar)
     int so;                           // sorted id (mtk: no row)
     bool live;                        // the item has this wave's block (wave-uniform)
@@ -170,7 +175,7 @@ __device__ __forceinline__ void items(
     r.so = w < it.nbk ? id : mtk;
     const int arow = r.so < mtk ? r.so / top_k : 0;
     r.va = WIDE ? arow : arow * K + 16 * c4;
-    r.vx = arow * nk + ksl;
+    r.vx = arow * nk;
     r.w0 = (it.set ? ws1 : ws) + ((size_t)it.e * (N / 128) + bcol(it.n0, 0) / 128) * nk;
     r.live = w < it.nbk;
     return r;
@@ -183,12 +188,14 @@ __device__ __forceinline__ void items(
       const uint8_t* p = qx + (size_t)r.va * K + c * KC * 128 + 16 * c4;
 #pragma unroll
       for (int ks = 0; ks < KC; ++ks) {
-        ra[ks][0] = *reinterpret_cast<const v4u*>(p + ks * 128);
-        ra[ks][1] = *reinterpret_cast<const v4u*>(p + ks * 128 + 64);
+        const int o = TAIL && c * KC + ks >= nk ? -c * KC * 128 : ks * 128;
+        ra[ks][0] = *reinterpret_cast<const v4u*>(p + o);
+        ra[ks][1] = *reinterpret_cast<const v4u*>(p + o + 64);
       }
     } else {
       const __amdgpu_buffer_rsrc_t q =
-          __builtin_amdgcn_make_buffer_rsrc((void*)qx, 0, r.live ? qbytes : 0, BUF_WORD3);
+          __builtin_amdgcn_make_buffer_rsrc((void*)qx, 0, r.live && (!TAIL || c * KC < nk) ? qbytes : 0,
+                                            BUF_WORD3);
 #pragma unroll
       for (int ks = 0; ks < KC; ++ks) {
         ra[ks][0] = __builtin_bit_cast(
@@ -197,9 +204,10 @@ __device__ __forceinline__ void items(
             v4u, __builtin_amdgcn_raw_buffer_load_b128(q, r.va + ks * 128 + 64, c * KC * 128, 0));
       }
     }
-    rx = xs[r.vx + c * KC];
-    rw0 = r.w0[c * KC + ksl];
-    rw1 = r.w0[c * KC + ksl + wrow];
+    const int k = TAIL ? min(c * KC + ksl, nk - 1) : c * KC + ksl;
+    rx = xs[r.vx + k];
+    rw0 = r.w0[k];
+    rw1 = r.w0[k + wrow];
     if (TWT) rt = tw[r.so < mtk ? r.so : 0];
   };
   unsigned abase[2], sbase[2];        // LDS byte addresses: [0] read, [1] written
@@ -249,10 +257,10 @@ __device__ __forceinline__ void items(
     rA = rows_of(mA, i0);
     rB = rows_of(mB, i1);
   }
-  __amdgpu_buffer_rsrc_t bcur = wbase(mA);
-  __amdgpu_buffer_rsrc_t bnext = wbase(mB);
+  const uint8_t* bcur = wptr(mA);
+  const uint8_t* bnext = wptr(mB);
 #pragma unroll
-  for (int j = 0; j < KC; ++j) issue_b(j, bcur, j * 2048);
+  for (int j = 0; j < KC; ++j) issue_b(j, wbuf(bcur, true), j * 2048);
   stage_a(rA, 0);
   write_a(rA);
   write_rows(rA, 0);
@@ -270,8 +278,10 @@ __device__ __forceinline__ void items(
       for (int s = 0; s < S; ++s) acc[bk][s] = v4f{0.f, 0.f, 0.f, 0.f};
     for (int c = 0; c < nch; ++c) {
       const bool last = c + 1 == nch;
-      const __amdgpu_buffer_rsrc_t bld = last ? bnext : bcur;
+      const uint8_t* bld = last ? bnext : bcur;
       const int woff = last ? 0 : (c + 1) * KC * 2048;
+      const int ahead = TAIL && !last ? nk - (c + 1) * KC : KC;   // steps of the next chunk
+      const int here = TAIL && last ? nk - c * KC : KC;           // ... of this one
       // the next chunk: this item's, or the next item's first
       Rows st = rA;
       if (last) st = rB;
@@ -330,6 +340,10 @@ __device__ __forceinline__ void items(
       rd(0, 0, abt, sbt);
 #pragma unroll
       for (int ks = 0; ks < KC; ++ks) {
+        if (TAIL && ks >= here) {                   // (uniform) the ring runs on
+          issue_b(ks, wbuf(bld, ks < ahead), woff + ks * 2048);
+          continue;
+        }
         if (r6) {
           unit(ks, 7, true);
           unit(ks, 6, false);
@@ -350,7 +364,7 @@ __device__ __forceinline__ void items(
         }
         unit(ks, 1, true);
         unit(ks, 0, false);
-        issue_b(ks, bld, woff + ks * 2048);
+        issue_b(ks, wbuf(bld, ks < ahead), woff + ks * 2048);
         scale(0);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -459,11 +473,11 @@ __device__ __forceinline__ void items(
     rA = rB;
     rB = rows_of(mB, idC);
     bcur = bnext;
-    bnext = wbase(mB);
+    bnext = wptr(mB);
   }
 }
 
-template <bool TWT, bool ACT, bool TWO, bool WIDE>
+template <bool TWT, bool ACT, bool TWO, bool WIDE, bool TAIL>
 __global__ __launch_bounds__(NWAVE * WAVE, 2) void roll_k(
     const uint8_t* __restrict__ qx, const float* __restrict__ xs, const uint8_t* __restrict__ wq,
     const float* __restrict__ ws, const int* __restrict__ sorted_ids,
@@ -479,11 +493,11 @@ __global__ __launch_bounds__(NWAVE * WAVE, 2) void roll_k(
   // two copies of the body: the policy is part of the load instructions, and a branch on it in
   // every step cost 2-5%
   if (sc.shared)
-    items<POL_SHARED, TWT, ACT, TWO, WIDE>(sc, qx, xs, wq, ws, sorted_ids, eids, wq1, ws1,
+    items<POL_SHARED, TWT, ACT, TWO, WIDE, TAIL>(sc, qx, xs, wq, ws, sorted_ids, eids, wq1, ws1,
                                            sorted_ids1, eids1, tiles, y, tw, q2, s2, mtk, top_k,
                                            K, N, qbytes);
   else
-    items<POL_STREAM, TWT, ACT, TWO, WIDE>(sc, qx, xs, wq, ws, sorted_ids, eids, wq1, ws1,
+    items<POL_STREAM, TWT, ACT, TWO, WIDE, TAIL>(sc, qx, xs, wq, ws, sorted_ids, eids, wq1, ws1,
                                            sorted_ids1, eids1, tiles, y, tw, q2, s2, mtk, top_k,
                                            K, N, qbytes);
 }
@@ -499,21 +513,27 @@ void launch_roll(const Args& a, int max_tiles, hipStream_t stream) {
   // bytes of the activation rows any id below mtk names; 32-bit offsets reach 2 GB of them
   const long long qbytes = (long long)((a.mtk + (long long)a.top_k - 1) / a.top_k) * a.K;
   const bool wide = qbytes > 0x7fffffff;
-#define RLU_PF1(T, A, TW, WD)                                                                 \
-  hipLaunchKernelGGL((roll_k<T, A, TW, WD>), dim3(grid), dim3(NWAVE * WAVE), LDS, stream, a.qx, \
-                     a.xs, a.wq, a.ws, a.sorted_ids, a.eids, a.wq1, a.ws1, a.sorted_ids1,       \
-                     a.eids1, a.tiles, a.ntiles, a.y, a.tw, a.q2, a.s2, a.mtk, a.top_k, a.K,    \
-                     a.N, wide ? 0 : (int)qbytes)
+  const bool tail = a.K % (KC * 128) != 0 || a.K < 2 * KC * 128;
+#define RLU_PF1(T, A, TW, WD, TL)                                                             \
+  hipLaunchKernelGGL((roll_k<T, A, TW, WD, TL>), dim3(grid), dim3(NWAVE * WAVE), LDS, stream,  \
+                     a.qx, a.xs, a.wq, a.ws, a.sorted_ids, a.eids, a.wq1, a.ws1,               \
+                     a.sorted_ids1, a.eids1, a.tiles, a.ntiles, a.y, a.tw, a.q2, a.s2, a.mtk,  \
+                     a.top_k, a.K, a.N, wide ? 0 : (int)qbytes)
+#define RLU_PF2(T, A, TW)                                                                     \
+  do {                                                                                        \
+    if (wide)                                       /* (the tail's code takes any K) */       \
+      RLU_PF1(T, A, TW, true, true);                                                          \
+    else if (tail)                                                                            \
+      RLU_PF1(T, A, TW, false, true);                                                         \
+    else                                                                                      \
+      RLU_PF1(T, A, TW, false, false);                                                        \
+  } while (0)
 #define RLU_PF(T, A)                                                                          \
   do {                                                                                        \
-    if (a.two && wide)                                                                        \
-      RLU_PF1(T, A, true, true);                                                              \
-    else if (a.two)                                                                           \
-      RLU_PF1(T, A, true, false);                                                             \
-    else if (wide)                                                                            \
-      RLU_PF1(T, A, false, true);                                                             \
+    if (a.two)                                                                                \
+      RLU_PF2(T, A, true);                                                                    \
     else                                                                                      \
-      RLU_PF1(T, A, false, false);                                                            \
+      RLU_PF2(T, A, false);                                                                   \
   } while (0)
   if (a.q2)
     RLU_PF(false, true);
@@ -522,6 +542,7 @@ void launch_roll(const Args& a, int max_tiles, hipStream_t stream) {
   else
     RLU_PF(false, false);
 #undef RLU_PF
+#undef RLU_PF2
 #undef RLU_PF1
 }
 

@@ -60,7 +60,7 @@ struct Item {
 
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 
-// The gate_up-shaped kernel of prefill_roll.hip; launched for K % 512 == 0, K >= 1024.
+// The gate_up-shaped kernel of prefill_roll.hip; launched for K % 128 == 0, K >= 512.
 void launch_roll(const Args& a, int max_tiles, hipStream_t stream);
 
 constexpr int ORD_MAX = 2048;   // tiles of one XCD's share that the LDS order holds

@@ -1,5 +1,4 @@
-"""The streamed prefill GEMMs (the unrolled K = 768 kernel and the rolled one for K a multiple of 512
-from 1024 on) against the general tiled kernel, which runs the same sequence of operations per
+"""The streamed prefill GEMMs (the unrolled K = 768 kernel and the rolled one for other K) against the general tiled kernel, which runs the same sequence of operations per
 output: equal bit for bit, over row distributions that take each branch of the tiles' schedule.
 """
 from __future__ import annotations
@@ -99,6 +98,18 @@ def test_streamed_equals_general_tiled(ops, name, K, N):
     check(ops, name, ROWS[name], K, N, routed=N % 512 == 0)
 
 
+# K of one chunk of 4 steps, with 1, 2 and 3 steps in the last one; these take the kernel from two
+# items per CU on (the row counts repeated until there are), and the general one below
+@pytest.mark.parametrize("K,N", [(512, 1536), (640, 2560), (1408, 2048), (1792, 1792)])
+@pytest.mark.parametrize("name", ["mixed", "alone", "shared", "thin", "mixed_few"])
+def test_streamed_broken_k_equals_general_tiled(ops, name, K, N):
+    rows = ROWS[name]
+    if name != "mixed_few":
+        cus = torch.cuda.get_device_properties(0).multi_processor_count
+        rows = rows * -(-2 * 128 * 256 * cus // (N * sum(rows)))
+    check(ops, name, rows, K, N, routed=name != "shared")
+
+
 @pytest.mark.parametrize("K", [768, 1024])
 @pytest.mark.parametrize("n", [16000, 16380, 17000])
 def test_streamed_at_the_orders_capacity(ops, n, K):
@@ -107,10 +118,11 @@ def test_streamed_at_the_orders_capacity(ops, n, K):
     check(ops, f"{n} tiles", [40] * n + [200], K, 256, routed=True, E=64)
 
 
-def test_streamed_activations_past_2gb(ops):
+@pytest.mark.parametrize("K", [2560, 2688])
+def test_streamed_activations_past_2gb(ops, K):
     """Row offsets past 31 bits take the 64-bit addresses: 2.2 GB of activations, of which the
     align names rows at both ends."""
-    tokens, K, N = 860_000, 2560, 256
+    tokens, N = 860_000, 256
     gen = torch.Generator(DEV).manual_seed(7)
     w, ws = weights(3, N, K, gen)
     qx = torch.randint(0, 0x7f, (tokens, K), dtype=torch.uint8, generator=gen,
