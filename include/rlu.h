@@ -357,6 +357,10 @@ int rlu_route_capture(const int* topk_ids, int n, int layer, int nlayer, int rin
  * -1 for a null pointer, else the launch status. */
 int rlu_selftest_bf16(unsigned long long* bad, hipStream_t stream);
 
+/* Likewise: the SiLU of the quantizing kernels against the float32 restatement the oracle follows,
+ * over all 2^16 bf16 inputs. */
+int rlu_selftest_silu(unsigned long long* bad, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

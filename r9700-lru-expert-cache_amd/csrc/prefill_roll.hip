@@ -448,7 +448,7 @@ __device__ __forceinline__ void items(
             uint32_t mx = 0;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-              a[j] = bf16_to_f32(f32_to_bf16_hw(__fmul_rn(silu_bf16_hw(gv[j]), uv[j])));
+              a[j] = bf16_to_f32(f32_to_bf16_hw(__fmul_rn(silu_of_bf16(gv[j]), uv[j])));
               mx = max(mx, abs_bits(a[j]));
             }
             const float sc = scale_of(row_max_u32(mx));

@@ -82,7 +82,7 @@ __global__ __launch_bounds__(QT) void silu_mul_quant_k(const uint16_t* __restric
     load8_bf16(g + c, gv);
     load8_bf16(u + c, uv);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) a[j] = bf16_to_f32(f32_to_bf16(__fmul_rn(silu_bf16(gv[j]), uv[j])));
+    for (int j = 0; j < 8; ++j) a[j] = bf16_to_f32(f32_to_bf16(__fmul_rn(silu_of_bf16(gv[j]), uv[j])));
     if (act) {
       uint32_t w[4];
 #pragma unroll
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(QT) void silu_mul_quant_g128_k(const uint16_t* __re
     uint32_t m = 0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      a[j] = bf16_to_f32(f32_to_bf16(__fmul_rn(silu_bf16(gv[j]), uv[j])));
+      a[j] = bf16_to_f32(f32_to_bf16(__fmul_rn(silu_of_bf16(gv[j]), uv[j])));
       m = max(m, abs_bits(a[j]));
     }
     const float s = scale_of(row_max_u32(m));
@@ -227,6 +227,13 @@ __global__ __launch_bounds__(SUM_THR) void moe_sum_k(const uint16_t* __restrict_
   *reinterpret_cast<uint4*>(out + (size_t)m * H + c) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// Self-test of silu_of_bf16: every bf16 bit pattern through both forms.
+__global__ __launch_bounds__(256) void silu_selftest_k(unsigned long long* __restrict__ bad) {
+  const float g = __uint_as_float((blockIdx.x * 256 + threadIdx.x) << 16);
+  const uint64_t m = __ballot(__float_as_uint(silu_of_bf16(g)) != __float_as_uint(silu_bf16(g)));
+  if (m && lane_id() == 0) atomicAdd(bad, (unsigned long long)__popcll(m));
+}
+
 // Self-test of f32_to_bf16_hw: every float32 bit pattern through both roundings; a thread
 // takes patterns 2 t and 2 t + 1 (opaque to the compiler, so nothing is folded between them)
 // and counts the patterns whose two results differ.
@@ -284,6 +291,15 @@ int rlu_moe_sum(const void* in, int M, int top_k, int H, void* out, hipStream_t 
   hipLaunchKernelGGL(rlu::moe_sum_k, dim3(M, (H + rlu::SUM_THR * 8 - 1) / (rlu::SUM_THR * 8)),
                      dim3(rlu::SUM_THR), 0, stream, (const uint16_t*)in, top_k, H,
                      (uint16_t*)out);
+  return (int)hipGetLastError();
+}
+
+// Counts the bf16 inputs (of all 2^16) on which silu_of_bf16 and silu_bf16 differ into *bad (which the
+// caller zeroes); 0 means they are interchangeable. Returns -1 for a null pointer, else the launch
+// status.
+int rlu_selftest_silu(unsigned long long* bad, hipStream_t stream) {
+  if (!bad) return -1;
+  hipLaunchKernelGGL(rlu::silu_selftest_k, dim3(256), dim3(256), 0, stream, bad);
   return (int)hipGetLastError();
 }
 
