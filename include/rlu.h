@@ -267,6 +267,21 @@ int rlu_moe_gemm_fp8blk_tiled_split_silu_quant(const void* qx, const float* xs, 
                                                float* s2, int mtk, int top_k, int K, int N,
                                                hipStream_t stream);
 
+/* The layer's form of the calls above, for every shape a streamed kernel takes (takes: 1 where one
+ * does for mtk rows; act: with the activation; K = 768 (plain only), a multiple of 512 from 1024 on,
+ * or any multiple of 128 from 512 on when mtk * N makes two 128 x 256 items per CU; N % 256 == 0).
+ * wq1 NULL: one align, tiles from rlu_moe_gemm_tiles; else two, from rlu_moe_gemm_tiles_split. q2
+ * NULL: y and topk_weights as rlu_moe_gemm_fp8blk_tiled; else q2 / s2 as _silu_quant (y and
+ * topk_weights NULL). Equal to those calls bit for bit. Returns -1 / -2 as they do, -6 for a shape
+ * that is not taken. */
+int rlu_moe_gemm_prefill_takes(int mtk, int K, int N, int act);
+int rlu_moe_gemm_prefill(const void* qx, const float* xs, const void* wq0, const float* ws0,
+                         const int* sorted_ids0, const int* expert_ids0, const void* wq1,
+                         const float* ws1, const int* sorted_ids1, const int* expert_ids1,
+                         const int* tiles, const int* ntiles, int max_tiles,
+                         const float* topk_weights, void* y, void* q2, float* s2, int mtk,
+                         int top_k, int K, int N, hipStream_t stream);
+
 /* No counterpart in the reference (which runs the down GEMM into ic3 and then vLLM's moe_sum,
  * r4d_mxfp4_moe.py.lru.diff:690-696): the decode down projection with moe_sum folded in.
  * out[t] (bf16 [M, N]) = sum over k in k order, in float32, of bf16(down row (t, k) x

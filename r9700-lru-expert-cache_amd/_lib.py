@@ -43,6 +43,8 @@ SIGNATURES: dict[str, tuple] = {
     "rlu_moe_gemm_fp8blk_tiled": (_I, [_P] * 8 + [_I, _P, _P] + [_I] * 5 + [_P]),
     "rlu_moe_gemm_fp8blk_tiled_noalloc": (_I, [_P] * 7 + [_I, _P, _P] + [_I] * 5 + [_P]),
     "rlu_moe_gemm_fp8blk_tiled_silu_quant": (_I, [_P] * 8 + [_I, _P, _P] + [_I] * 4 + [_P]),
+    "rlu_moe_gemm_prefill_takes": (_I, [_I] * 4),
+    "rlu_moe_gemm_prefill": (_I, [_P] * 12 + [_I] + [_P] * 4 + [_I] * 4 + [_P]),
     "rlu_moe_gemm_tiles_split": (_I, [_P, _P, _I, _P, _P, _I, _P, _P, _P]),
     "rlu_moe_gemm_fp8blk_tiled_split": (_I, [_P] * 12 + [_I, _P, _P] + [_I] * 4 + [_P]),
     "rlu_moe_gemm_fp8blk_tiled_split_silu_quant": (_I, [_P] * 12 + [_I, _P, _P] + [_I] * 4 +

@@ -402,6 +402,37 @@ int rlu_moe_gemm_fp8blk_tiled_silu_quant(const void* qx, const float* xs, const 
 
 // ---- two aligns in one launch (a layer's resident slots and its non-resident experts) ------
 
+// One launch of a streamed kernel for a layer's prefill: set 0 alone (wq1 NULL) or sets 0 and 1 with
+// the list of both, y or (with q2) the activation's bytes and scales.
+int rlu_moe_gemm_prefill_takes(int mtk, int K, int N, int act) {
+  return mtk > 0 && rlu::prefill_stream_takes(mtk, K, N, act != 0) ? 1 : 0;
+}
+
+int rlu_moe_gemm_prefill(const void* qx, const float* xs, const void* wq0, const float* ws0,
+                         const int* sorted_ids0, const int* expert_ids0, const void* wq1,
+                         const float* ws1, const int* sorted_ids1, const int* expert_ids1,
+                         const int* tiles, const int* ntiles, int max_tiles,
+                         const float* topk_weights, void* y, void* q2, float* s2, int mtk,
+                         int top_k, int K, int N, hipStream_t stream) {
+  using namespace rlu::tiled;
+  const int rc = check_gemm_args(mtk, top_k, K, N, max_tiles, 0);
+  if (rc) return rc;
+  if (mtk == 0) return 0;
+  if (!rlu::prefill_stream_takes(mtk, K, N, q2 != nullptr)) return -6;
+  if (!qx || !xs || !wq0 || !ws0 || !sorted_ids0 || !expert_ids0 || !tiles || !ntiles ||
+      (q2 ? !s2 || topk_weights : !y) || (wq1 && (!ws1 || !sorted_ids1 || !expert_ids1)))
+    return -1;
+  const rlu::PfSecond second{wq1, ws1, sorted_ids1, expert_ids1};
+  const rlu::PfSecond* b = wq1 ? &second : nullptr;
+  if (q2 ? rlu::launch_prefill_stream_act(qx, xs, wq0, ws0, sorted_ids0, expert_ids0, b, tiles,
+                                          ntiles, max_tiles, q2, s2, mtk, top_k, K, N, stream)
+         : rlu::launch_prefill_stream(qx, xs, wq0, ws0, sorted_ids0, expert_ids0, b, tiles,
+                                      ntiles, max_tiles, topk_weights, y, mtk, top_k, K, N,
+                                      stream))
+    return -6;
+  return (int)hipGetLastError();
+}
+
 // The tile list of both aligns: align 0's tiles, then align 1's with bit 16 of the block
 // count set. tiles holds 2 (nb_max0 + nb_max1) ints.
 int rlu_moe_gemm_tiles_split(const int* expert_ids0, const int* num_post_pad0, int nb_max0,

@@ -14,8 +14,11 @@ struct PfSecond {
   const int* expert_ids;
 };
 
-// K and N of the two-set launches.
+// K and N of the two-set entry points.
 bool prefill_stream_built(int K, int N);
+
+// Whether the launches below take mtk rows of this shape (act: the one with the activation).
+bool prefill_stream_takes(int mtk, int K, int N, bool act);
 
 // Launches a streamed kernel over a tile list (tiles of <= 8 blocks) when one takes K and N (K =
 // 768, or what roll_takes says, N % 256 == 0), and returns 0; returns -1 (nothing
@@ -28,7 +31,7 @@ int launch_prefill_stream(const void* qx, const float* xs, const void* wq, const
 
 // The same kernel for gate_up with SiLU-mul-quant in its epilogue: writes q2 [mtk, N / 2] e4m3
 // and s2 [mtk, N / 256] (group-128 scales) instead of the bf16 output. Returns -1 (nothing
-// launched) when K and N have no built configuration.
+// launched) where roll_takes says no; prefill_stream_act_built: the shapes of its entry points.
 bool prefill_stream_act_built(int K, int N);
 int launch_prefill_stream_act(const void* qx, const float* xs, const void* wq, const float* ws,
                               const int* sorted_ids, const int* expert_ids,

@@ -402,7 +402,7 @@ bool prefill_stream_built(int K, int N) { return (K == 2560 || K == 768) && N % 
 // up for less of that (32 experts, 512 tokens, K = 896: 52 against 46 us of tiled_k; 256 experts, 64
 // tokens, K = 512: 45 against 39).
 static bool roll_takes(int mtk, int K, int N) {
-  if (K % 128 || K < 512) return false;
+  if (K % 128 || K < 512 || N % 256) return false;
   return (K % 512 == 0 && K >= 1024) ||
          (long long)mtk * N >= 2LL * 16 * pf::TB * 256 * device_cus();
 }
@@ -426,12 +426,16 @@ int launch_prefill_stream(const void* qx, const float* xs, const void* wq, const
 
 bool prefill_stream_act_built(int K, int N) { return K == 2560 && N % 256 == 0; }
 
+bool prefill_stream_takes(int mtk, int K, int N, bool act) {
+  return (!act && K == 768 && N % 256 == 0) || roll_takes(mtk, K, N);
+}
+
 int launch_prefill_stream_act(const void* qx, const float* xs, const void* wq, const float* ws,
                               const int* sorted_ids, const int* expert_ids,
                               const PfSecond* second, const int* tiles, const int* ntiles,
                               int max_tiles, void* q2, float* s2, int mtk, int top_k, int K,
                               int N, hipStream_t stream) {
-  if (!prefill_stream_act_built(K, N)) return -1;
+  if (!roll_takes(mtk, K, N)) return -1;
   const pf::Args a = make_args(qx, xs, wq, ws, sorted_ids, expert_ids, second, tiles, ntiles,
                                nullptr, nullptr, q2, s2, mtk, top_k, K, N);
   pf::launch_roll(a, max_tiles, stream);

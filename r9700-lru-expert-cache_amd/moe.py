@@ -149,9 +149,10 @@ class LruMoELayer:
                         and top_k == 10 and self.cache.max_inserts > 0)
         self.fold_sum = fold_sum
         self.ids32 = torch.empty((self.M, top_k), dtype=torch.int32, device=dev)
-        # prefill gate_up with SiLU-mul-quant in its epilogue where a kernel is built for the
+        # prefill gate_up with SiLU-mul-quant in its epilogue where a streamed kernel takes the
         # shape: no [mtk, 2I] bf16 intermediate (same q2 / s2 bits)
-        self.fuse_act = self.prefill and ops.moe_gemm_tiled_silu_quant_built(self.H, self.N1)
+        self.fuse_act = self.prefill and ops.moe_gemm_prefill_takes(self.mtk, self.H, self.N1,
+                                                                    act=True)
         # decode: gate_up with its activation, down quantizing it (no activation launch)
         if fuse_act is None:
             fuse_act = (not self.prefill and npw1 == 2 and npw2 == 4 and sk2 == 1 and wv == 0
@@ -172,11 +173,13 @@ class LruMoELayer:
             self.tiles = {t.data_ptr(): torch.empty(2 * t.numel() + 1, dtype=torch.int32,
                                                     device=dev)
                           for t in (self.align[1], self.align[4], self.eids_res, self.eids_new)}
-            # where the streamed kernel is built for both GEMMs, a GEMM over the hot align (or
-            # the overlap's resident bucket) and the cold align is one launch over one tile
-            # list of both (an empty cold align then costs no launch of its own)
-            self.pf_split = (ops.moe_gemm_tiled_split_built(self.H, self.N1) and
-                             ops.moe_gemm_tiled_split_built(self.I, self.H))
+            # where streamed kernels take both GEMMs, a GEMM over the hot align (or the
+            # overlap's resident bucket) and the cold align is one launch over one tile list
+            # of both (an empty cold align then costs no launch of its own; with the
+            # activation in gate_up a 2048-token step over 128 experts of hidden 2048 takes
+            # 270 us, in separate launches 278)
+            self.pf_split = (ops.moe_gemm_prefill_takes(self.mtk, self.H, self.N1) and
+                             ops.moe_gemm_prefill_takes(self.mtk, self.I, self.H))
             ec = self.align[4]
             self.split_tiles = {
                 (t.data_ptr(), ec.data_ptr()): torch.empty(2 * (t.numel() + ec.numel()) + 1,
@@ -268,9 +271,9 @@ class LruMoELayer:
         if self.prefill:
             full = self.full.tensors()
             if self.pf_split:
-                ops.moe_gemm_tiled_split(y, qx, xs, slot_w, slot_s, (sh, eh, nh), full[part],
-                                         full[part + 1], (sc, ec, nc), tw, y.shape[0], top_k,
-                                         tiles=self._split_tiles_of(eh, nh), tiles_ready=True)
+                ops.moe_gemm_prefill(y, qx, xs, slot_w, slot_s, (sh, eh, nh),
+                                     (full[part], full[part + 1], (sc, ec, nc)), tw, y.shape[0],
+                                     top_k, self._split_tiles_of(eh, nh))
                 return
             self._gemm_tiled(y, qx, xs, slot_w, slot_s, sh, eh, nh, tw, top_k)
             self._gemm_tiled(y, qx, xs, full[part], full[part + 1], sc, ec, nc, tw, top_k)
@@ -338,17 +341,15 @@ class LruMoELayer:
             sh, eh0, nh, sc, ec, nc = self.align
             eh = eh0 if eh is None else eh
             if cold and self.pf_split:
-                ops.moe_gemm_tiled_split_silu_quant(
-                    self.q2, self.s2, self.qx, self.xs, self.slots.w13, self.slots.s13,
-                    (sh, eh, nh), self.full.w13, self.full.s13, (sc, ec, nc), self.mtk,
-                    self.top_k, tiles=self._split_tiles_of(eh, nh), tiles_ready=True)
+                ops.moe_gemm_prefill(
+                    (self.q2, self.s2), self.qx, self.xs, self.slots.w13, self.slots.s13,
+                    (sh, eh, nh), (self.full.w13, self.full.s13, (sc, ec, nc)), None, self.mtk,
+                    self.top_k, self._split_tiles_of(eh, nh))
                 return
             for w, s, al in (((self.slots.w13, self.slots.s13, (sh, eh, nh)),) +
                              (((self.full.w13, self.full.s13, (sc, ec, nc)),) if cold else ())):
-                ops.moe_gemm_tiled_silu_quant(self.q2, self.s2, self.qx, self.xs, w, s, *al,
-                                              self.mtk, self.top_k,
-                                              tiles=self._tiles_of(al[1], al[2]),
-                                              tiles_ready=True)
+                ops.moe_gemm_prefill((self.q2, self.s2), self.qx, self.xs, w, s, al, None, None,
+                                     self.mtk, self.top_k, self._tiles_of(al[1], al[2]))
             return
         up = (self.ic1, self.qx, self.xs, self.slots.w13, self.slots.s13)
         if cold:

@@ -464,6 +464,42 @@ def moe_gemm_tiled_split_silu_quant(q2: torch.Tensor, s2: torch.Tensor, qx: torc
     check(rc, "rlu_moe_gemm_fp8blk_tiled_split_silu_quant")
 
 
+def moe_gemm_prefill_takes(mtk: int, K: int, N: int, act: bool = False) -> bool:
+    """Whether moe_gemm_prefill has a kernel for mtk rows of weights [*, N, K] (act: with q2)."""
+    return lib().rlu_moe_gemm_prefill_takes(mtk, K, N, int(act)) == 1
+
+
+def moe_gemm_prefill(out, qx: torch.Tensor, x_scale: torch.Tensor, w0: torch.Tensor,
+                     s0: torch.Tensor, al0, second, topk_weights: torch.Tensor | None, mtk: int,
+                     top_k: int, tiles: torch.Tensor) -> None:
+    """A layer's prefill GEMM in one launch of a streamed kernel: al0 = (sorted_ids, expert_ids,
+    num_post_pad) over w0 / s0 alone (second None; tiles = moe_gemm_tiles) or with second = (w1,
+    s1, al1) (tiles = moe_gemm_tiles_split). out is y, as moe_gemm_tiled(_split), or (q2, s2), as
+    their _silu_quant forms; equal to them bit for bit."""
+    N, K = w0.shape[1:]
+    q2, s2 = out if isinstance(out, tuple) else (None, None)
+    y = out if q2 is None else None
+    if q2 is None:
+        assert y.shape == (mtk, N) and y.dtype == torch.bfloat16 and y.is_contiguous()
+    else:
+        assert q2.shape == (mtk, N // 2) and q2.dtype == FP8 and q2.is_contiguous()
+        assert s2.shape == (mtk, N // 256) and s2.dtype == torch.float32 and s2.is_contiguous()
+    assert qx.dtype == FP8 and w0.dtype == FP8 and qx.shape[1] == K
+    nb = al0[1].numel()
+    b = [_P(0)] * 4
+    if second is not None:
+        w1, s1, al1 = second
+        assert w1.dtype == FP8 and w1.shape[1:] == (N, K)
+        nb += al1[1].numel()
+        b = [_P(device_ptr(w1)), _P(device_ptr(s1)), _p(al1[0]), _p(al1[1])]
+    assert tiles.numel() == 2 * nb + 1 and tiles.dtype == torch.int32
+    rc = lib().rlu_moe_gemm_prefill(
+        _p(qx), _p(x_scale), _P(device_ptr(w0)), _P(device_ptr(s0)), _p(al0[0]), _p(al0[1]), *b,
+        _p(tiles), _P(tiles.data_ptr() + 8 * nb), nb, _p(topk_weights), _p(y), _p(q2), _p(s2),
+        mtk, top_k, K, N, _P(stream_ptr()))
+    check(rc, "rlu_moe_gemm_prefill")
+
+
 NOALLOC_MAX_BLOCKS = 8192      # the scratch tile list's capacity (131072 sorted ids)
 
 

@@ -33,9 +33,9 @@ ROWS = {
 SHAPES = [(768, 512), (1024, 256), (1536, 256), (2048, 768), (2560, 512), (4096, 256)]
 
 
-def align(rows, order):
-    """One align of mtk = sum(rows) ids dealt to the experts in the given order."""
-    mtk = sum(rows)
+def align(rows, order, mtk=None):
+    """One align of sum(rows) ids dealt to the experts in the given order, padded with mtk."""
+    mtk = sum(rows) if mtk is None else mtk
     sid, eid, pos = [], [], 0
     for e, r in enumerate(rows):
         nb = (r + 15) // 16
@@ -140,3 +140,58 @@ def test_streamed_activations_past_2gb(ops, K):
         torch.cuda.synchronize()
         out.append(y.view(torch.int16))
     assert torch.equal(*out) and bool(out[0][ids].any())
+
+
+# whole and broken K; few items (the broken K then has no kernel) and two per CU
+@pytest.mark.parametrize("two", [False, True])
+@pytest.mark.parametrize("K,I,rep", [(1024, 256, 1), (2048, 384, 1), (640, 640, 4), (1408, 512, 6)])
+def test_layer_prefill_gemm_equals_its_parts(ops, K, I, rep, two):
+    """moe_gemm_prefill (one or two aligns; plain with routed weights, or with the activation) against
+    the general tiled kernel on each align and silu_mul_quant."""
+    N, rows = 2 * I, ROWS["mixed"] * rep
+    gen = torch.Generator(DEV).manual_seed(K + I)
+    rows1 = [r if i % 3 else 0 for i, r in enumerate(rows)] if two else rows
+    rows2 = [r - q for r, q in zip(rows, rows1)]
+    mtk = sum(rows)
+    assert ops.moe_gemm_prefill_takes(mtk, K, N) and ops.moe_gemm_prefill_takes(mtk, K, N, True)
+    order = torch.randperm(mtk, generator=torch.Generator().manual_seed(2)).tolist()
+    sets = []
+    for rs, o in ((rows1, order[:sum(rows1)]), (rows2, order[sum(rows1):]))[:1 + two]:
+        sets.append((*weights(len(rows), N, K, gen), align(rs, o, mtk)))
+    qx = torch.randint(0, 0x7f, (mtk, K), dtype=torch.uint8, generator=gen, device=DEV)
+    qx = (qx ^ 0x80 * (qx & 1)).view(torch.float8_e4m3fn)
+    xs = torch.rand(mtk, K // 128, generator=gen, device=DEV)
+    tw = torch.rand(mtk, generator=gen, device=DEV)
+    (w, s, al), second = sets[0], (sets[1] if two else None)
+    tiles = ops.moe_gemm_tiles_split(al[1:], second[2][1:]) if two else ops.moe_gemm_tiles(*al[1:])
+    gpu_case(f"layer prefill gemm K={K} N={N} two={two}")
+    want, routed = (torch.empty(mtk, N, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    for w_, s_, al_ in sets:
+        ops.moe_gemm_tiled(want, qx, xs, w_, s_, *al_, None, mtk, 1, wv=2)
+        ops.moe_gemm_tiled(routed, qx, xs, w_, s_, *al_, tw, mtk, 1, wv=2)
+    q0, s0 = ops.silu_mul_quant(want, group=128)[1:]
+    y = torch.empty_like(want)
+    q2, s2 = torch.empty_like(q0), torch.empty_like(s0)
+    ops.moe_gemm_prefill(y, qx, xs, w, s, al, second, tw, mtk, 1, tiles)
+    ops.moe_gemm_prefill((q2, s2), qx, xs, w, s, al, second, None, mtk, 1, tiles)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), routed.view(torch.int16))
+    assert torch.equal(q2.view(torch.uint8), q0.view(torch.uint8)) and torch.equal(s2, s0)
+
+
+def test_layer_prefill_gemm_shapes_and_return_codes(pkg, ops):
+    import ctypes
+    P = ctypes.c_void_p
+    takes = ops.moe_gemm_prefill_takes
+    assert takes(1, 2560, 1536, True) and takes(1, 768, 2560) and not takes(1, 768, 2560, True)
+    assert takes(1, 1024, 256) and not takes(1, 1024, 384) and not takes(0, 2560, 1536)
+    assert not takes(4096, 640, 256) and not takes(1 << 20, 384, 2048)
+    assert not takes(1 << 20, 1000, 2048)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert takes(256 * cus, 640, 256) and not takes(256 * cus - 1, 640, 256)
+    f, s = pkg.lib().rlu_moe_gemm_prefill, P(torch.cuda.current_stream().cuda_stream)
+    z = P(0)
+    call = lambda mtk, K, N, y, q: f(*([z] * 12), 1, z, y, q, z, mtk, 1, K, N, s)
+    assert call(20, 2560, 1536, z, z) == -1 and call(20, 384, 1536, z, z) == -6
+    assert call(20, 768, 2560, z, P(1)) == -6 and call(20, 2560, 1500, z, z) == -2
+    assert call(0, 2560, 1536, z, z) == 0
