@@ -376,6 +376,11 @@ int rlu_selftest_bf16(unsigned long long* bad, hipStream_t stream);
  * over all 2^16 bf16 inputs. */
 int rlu_selftest_silu(unsigned long long* bad, hipStream_t stream);
 
+/* On the host, without a GPU: the loads of activation rows, over the first and the last of `rows`
+ * rows of K bytes, by which the rolled prefill kernel would touch memory outside of its row. Returns
+ * 0, -1 (bad sizes or NULL), -2 (K % 128, K < 512, or rows * K past 2 GB). */
+int rlu_selftest_prefill_rows(int rows, int K, unsigned long long* bad);
+
 #ifdef __cplusplus
 }
 #endif

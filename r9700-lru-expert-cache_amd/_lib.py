@@ -54,6 +54,7 @@ SIGNATURES: dict[str, tuple] = {
     "rlu_route_capture": (_I, [_P] + [_I] * 5 + [_P] * 4),
     "rlu_selftest_bf16": (_I, [_P, _P]),
     "rlu_selftest_silu": (_I, [_P, _P]),
+    "rlu_selftest_prefill_rows": (_I, [_I, _I, _P]),
 }
 
 

@@ -31,6 +31,7 @@
 #include "numerics.h"
 #include "prefill_sched.h"
 #include "quant_row.h"
+#include "rlu.h"
 #include "wave.h"
 
 namespace rlu {
@@ -64,6 +65,31 @@ __device__ __forceinline__ float quad(float x) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), I * 0x55, 0xf, 0xf, true));
 }
 
+// Chunks of an item of nk steps. TAIL: the last chunk has what KC leaves of them, nothing where they
+// are one chunk alone (the metadata pipeline takes two). (max and no branch: on one, the compiler
+// copies the loop for two chunks and spills 155-202 registers.)
+template <bool TAIL>
+__host__ __device__ __forceinline__ int chunks(int nk) {
+  return TAIL ? max(2, (nk + KC - 1) / KC) : nk / KC;
+}
+inline bool has_tail(int K) { return K % (KC * 128) != 0 || K < 2 * KC * 128; }
+
+// Chunk c's loads of one lane's row, byte va of qbytes bytes of activations on: ld(ks, h, bytes,
+// voffset, soffset) reads 16 bytes through a buffer of `bytes`, zeros where voffset is past it. Only
+// the vector offset is sure to count in a buffer's range check, so a step that K does not have
+// (TAIL) and every step of a block that the tile does not have take an empty buffer, instead of
+// reading on: into the next row, and behind the last one past the tensor.
+template <bool TAIL, class LD>
+__host__ __device__ __forceinline__ void row_loads(int qbytes, int nk, int va, int c, bool live,
+                                                   const LD& ld) {
+#pragma unroll
+  for (int ks = 0; ks < KC; ++ks) {
+    const int bytes = live && (!TAIL || c * KC + ks < nk) ? qbytes : 0;
+    ld(ks, 0, bytes, va + ks * 128, c * KC * 128);
+    ld(ks, 1, bytes, va + ks * 128 + 64, c * KC * 128);
+  }
+}
+
 // ACT: SiLU-mul-quant in the epilogue. N = 2 I (gate | up); item g covers gate columns [128 g,
 // 128 g + 128) (waves 0 .. 3) and the matching up columns [I + 128 g, ...) (waves 4 .. 7), so
 // each output row's 128-column activation group is whole in one item. The epilogue writes q2
@@ -92,9 +118,7 @@ __device__ __forceinline__ void items(
   const int r16 = lane & 15, c4 = lane >> 4;
   const int cb = w / (NWAVE / 2);                       // this wave's 128-column scale block
   const int nk = K / 128;
-  // TAIL: the last chunk has what KC leaves of K / 128, nothing where that is one chunk alone (the
-  // metadata pipeline takes two)
-  const int nch = TAIL ? max(2, (nk + KC - 1) / KC) : nk / KC;
+  const int nch = chunks<TAIL>(nk);
   const int ncg = N / C;
   // first output column of scale block h of an item starting at column n0
   auto bcol = [&](int n0, int h) __attribute__((always_inline)) -> int {
@@ -180,9 +204,9 @@ __device__ __forceinline__ void items(
     r.live = w < it.nbk;
     return r;
   };
-  // Chunk c of an item's rows and scales. Without its block a wave reads through an empty buffer,
-  // so that no memory is touched (at one block per tile the rows of the other seven waves cost
-  // 2-4 us of 28 per item). WIDE: activations past 2 GB take 64-bit addresses, not a buffer.
+  // Chunk c of an item's rows and scales. Without its block a wave reads through empty buffers
+  // (row_loads): at one block per tile the rows of the other seven waves cost 2-4 us of 28 per
+  // item. WIDE: activations past 2 GB take 64-bit addresses, not a buffer.
   auto stage_a = [&](const Rows& r, int c) __attribute__((always_inline)) {
     if constexpr (WIDE) {
       const uint8_t* p = qx + (size_t)r.va * K + c * KC * 128 + 16 * c4;
@@ -193,16 +217,14 @@ __device__ __forceinline__ void items(
         ra[ks][1] = *reinterpret_cast<const v4u*>(p + o + 64);
       }
     } else {
-      const __amdgpu_buffer_rsrc_t q =
-          __builtin_amdgcn_make_buffer_rsrc((void*)qx, 0, r.live && (!TAIL || c * KC < nk) ? qbytes : 0,
-                                            BUF_WORD3);
-#pragma unroll
-      for (int ks = 0; ks < KC; ++ks) {
-        ra[ks][0] = __builtin_bit_cast(
-            v4u, __builtin_amdgcn_raw_buffer_load_b128(q, r.va + ks * 128, c * KC * 128, 0));
-        ra[ks][1] = __builtin_bit_cast(
-            v4u, __builtin_amdgcn_raw_buffer_load_b128(q, r.va + ks * 128 + 64, c * KC * 128, 0));
-      }
+      row_loads<TAIL>(qbytes, nk, r.va, c, r.live,
+                      [&](int ks, int h, int bytes, int voffset, int soffset)
+                          __attribute__((always_inline)) {
+        ra[ks][h] = __builtin_bit_cast(
+            v4u, __builtin_amdgcn_raw_buffer_load_b128(
+                     __builtin_amdgcn_make_buffer_rsrc((void*)qx, 0, bytes, BUF_WORD3), voffset,
+                     soffset, 0));
+      });
     }
     const int k = TAIL ? min(c * KC + ksl, nk - 1) : c * KC + ksl;
     rx = xs[r.vx + k];
@@ -502,6 +524,23 @@ __global__ __launch_bounds__(NWAVE * WAVE, 2) void roll_k(
                                            K, N, qbytes);
 }
 
+// row_loads' 16-byte loads, over the first and the last of `rows` rows of K bytes, that reach bytes
+// outside of their own row
+template <bool TAIL>
+static int loads_outside(int rows, int K) {
+  int bad = 0;
+  for (int row : {0, rows - 1})
+    for (int c4 = 0; c4 < 4; ++c4)
+      for (int live = 0; live < 2; ++live)
+        for (int c = 0; c < chunks<TAIL>(K / 128); ++c)
+          row_loads<TAIL>(rows * K, K / 128, row * K + 16 * c4, c, live != 0,
+                          [&](int, int, int bytes, int voffset, int soffset) {
+            const long long at = (long long)voffset + soffset - (long long)row * K;
+            if (voffset < bytes && (!live || at < 0 || at + 16 > K)) ++bad;
+          });
+  return bad;
+}
+
 }  // namespace roll
 
 void launch_roll(const Args& a, int max_tiles, hipStream_t stream) {
@@ -513,7 +552,7 @@ void launch_roll(const Args& a, int max_tiles, hipStream_t stream) {
   // bytes of the activation rows any id below mtk names; 32-bit offsets reach 2 GB of them
   const long long qbytes = (long long)((a.mtk + (long long)a.top_k - 1) / a.top_k) * a.K;
   const bool wide = qbytes > 0x7fffffff;
-  const bool tail = a.K % (KC * 128) != 0 || a.K < 2 * KC * 128;
+  const bool tail = has_tail(a.K);
 #define RLU_PF1(T, A, TW, WD, TL)                                                             \
   hipLaunchKernelGGL((roll_k<T, A, TW, WD, TL>), dim3(grid), dim3(NWAVE * WAVE), LDS, stream,  \
                      a.qx, a.xs, a.wq, a.ws, a.sorted_ids, a.eids, a.wq1, a.ws1,               \
@@ -548,3 +587,15 @@ void launch_roll(const Args& a, int max_tiles, hipStream_t stream) {
 
 }  // namespace pf
 }  // namespace rlu
+
+// Host only: counts into *bad the loads of activation rows by which the rolled kernel would touch
+// bytes outside of its row, over the first and the last of `rows` rows of K, with only the vector
+// offset in the buffers' range check. Returns -1 (bad sizes or NULL), -2 (K % 128, K < 512, or
+// activations past 2 GB, which take 64-bit addresses).
+extern "C" int rlu_selftest_prefill_rows(int rows, int K, unsigned long long* bad) {
+  using namespace rlu::pf::roll;
+  if (rows < 1 || K < 1 || !bad) return -1;
+  if (K % 128 || K < 512 || (long long)rows * K > 0x7fffffff) return -2;
+  *bad = has_tail(K) ? loads_outside<true>(rows, K) : loads_outside<false>(rows, K);
+  return 0;
+}
