@@ -342,10 +342,10 @@ __global__ __launch_bounds__(W * WAVE, 2) void stream_k(
     const int* __restrict__ eids, const uint8_t* __restrict__ wq1, const float* __restrict__ ws1,
     const int* __restrict__ sorted_ids1, const int* __restrict__ eids1,
     const int* __restrict__ tiles, const int* __restrict__ ntiles, uint16_t* __restrict__ y,
-    const float* __restrict__ tw, int mtk, int top_k, int N) {
+    const float* __restrict__ tw, int mtk, int top_k, int N, bool far) {
   extern __shared__ __align__(16) unsigned char smem[];
   const Sched sc = make_sched<TWO>(smem, smem + ORD_OFF, tiles, ntiles[0], mtk, N / C, eids,
-                                  eids1);
+                                  eids1, far);
   if (sc.first >= sc.n * (N / C)) return;
   if (sc.shared)                                    // two copies: the policy is in the loads
     items<POL_SHARED, TWT, TWO>(sc, qx, xs, wq, ws, sorted_ids, eids, wq1, ws1, sorted_ids1,
@@ -366,7 +366,7 @@ static void launch_k768(const Args& a, int max_tiles, hipStream_t stream) {
 #define RLU_PF(T, TW)                                                                         \
   hipLaunchKernelGGL((stream_k<T, TW>), dim3(grid), dim3(W * WAVE), LDS, stream, a.qx, a.xs,  \
                      a.wq, a.ws, a.sorted_ids, a.eids, a.wq1, a.ws1, a.sorted_ids1, a.eids1,  \
-                     a.tiles, a.ntiles, a.y, a.tw, a.mtk, a.top_k, a.N)
+                     a.tiles, a.ntiles, a.y, a.tw, a.mtk, a.top_k, a.N, a.far)
   if (a.tw && a.two)
     RLU_PF(true, true);
   else if (a.tw)
@@ -380,6 +380,14 @@ static void launch_k768(const Args& a, int max_tiles, hipStream_t stream) {
 
 }  // namespace pf
 
+// Whether p is the device address of pinned host memory (no: memory the runtime does not know)
+static bool in_host_memory(const void* p) {
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type == hipMemoryTypeHost;
+  (void)hipGetLastError();                          // the entry points return the launch's status
+  return false;
+}
+
 // the kernel arguments; without a second set, set 1 repeats set 0 (no tile names it)
 static pf::Args make_args(const void* qx, const float* xs, const void* wq, const float* ws,
                           const int* sorted_ids, const int* expert_ids, const PfSecond* second,
@@ -389,7 +397,7 @@ static pf::Args make_args(const void* qx, const float* xs, const void* wq, const
   const PfSecond& b = second ? *second : one;
   return pf::Args{(const uint8_t*)qx, xs, (const uint8_t*)wq, ws, sorted_ids, expert_ids,
                   (const uint8_t*)b.wq, b.ws, b.sorted_ids, b.expert_ids, second != nullptr,
-                  tiles, ntiles,
+                  second && in_host_memory(b.wq), tiles, ntiles,
                   (uint16_t*)y, topk_weights, (uint8_t*)q2, s2, mtk, top_k, K, N};
 }
 

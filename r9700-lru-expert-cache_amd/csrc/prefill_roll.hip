@@ -507,10 +507,10 @@ __global__ __launch_bounds__(NWAVE * WAVE, 2) void roll_k(
     const int* __restrict__ sorted_ids1, const int* __restrict__ eids1,
     const int* __restrict__ tiles, const int* __restrict__ ntiles, uint16_t* __restrict__ y,
     const float* __restrict__ tw, uint8_t* __restrict__ q2, float* __restrict__ s2, int mtk,
-    int top_k, int K, int N, int qbytes) {
+    int top_k, int K, int N, int qbytes, bool far) {
   extern __shared__ __align__(16) unsigned char smem[];
   const Sched sc = make_sched<TWO>(smem, smem + ORD_OFF, tiles, ntiles[0], mtk, N / C, eids,
-                                  eids1);
+                                  eids1, far);
   if (sc.first >= sc.n * (N / C)) return;
   // two copies of the body: the policy is part of the load instructions, and a branch on it in
   // every step cost 2-5%
@@ -557,7 +557,7 @@ void launch_roll(const Args& a, int max_tiles, hipStream_t stream) {
   hipLaunchKernelGGL((roll_k<T, A, TW, WD, TL>), dim3(grid), dim3(NWAVE * WAVE), LDS, stream,  \
                      a.qx, a.xs, a.wq, a.ws, a.sorted_ids, a.eids, a.wq1, a.ws1,               \
                      a.sorted_ids1, a.eids1, a.tiles, a.ntiles, a.y, a.tw, a.q2, a.s2, a.mtk,  \
-                     a.top_k, a.K, a.N, wide ? 0 : (int)qbytes)
+                     a.top_k, a.K, a.N, wide ? 0 : (int)qbytes, a.far)
 #define RLU_PF2(T, A, TW)                                                                     \
   do {                                                                                        \
     if (wide)                                       /* (the tail's code takes any K) */       \

@@ -42,6 +42,7 @@ struct Args {
   const int* sorted_ids1;
   const int* eids1;
   bool two;                      // a two-set tile list
+  bool far;                      // ... of which the second set is in host memory
   const int* tiles;
   const int* ntiles;
   uint16_t* y;
@@ -97,11 +98,19 @@ constexpr int SPLIT_ROWS = 24;
 // two lists by cost (ncg: column groups, items per tile). scratch: SCRATCH_BYTES of LDS that the
 // kernel does not use yet; ord: ORD_BYTES that it keeps. List order, an equal share of the tiles
 // per XCD, where there is nothing to split.
+// far: a two-set list's second set is in host memory. Its tiles wait for the host link, for fifty times
+// as long as all the others together, and they stand behind the first set's, so in list order each
+// XCD leaves the link idle until its unshared tiles of the first set are done: the unshared tiles
+// are then walked from the end. 512 experts, 257 of them resident, 2048 / 4096 tokens: 28.2 ->
+// 27.2 / 27.5 ms (unsplit, 27.6 / 27.5); 128 experts, 65 resident, 617 / 4096 tokens: 6.59 -> 5.51 /
+// 5.71 -> 5.45 ms (unsplit 6.45 / 6.78). From both ends in turn: 28.0 / 27.8, 6.15 / 5.71. With both
+// sets in HBM the reverse order costs 1-3% (2048 tokens 686 -> 704 us): the resident experts'
+// larger tiles then come last.
 template <bool TWO>
 __device__ __forceinline__ Sched make_sched(unsigned char* scratch, unsigned char* ord,
                                             const int* __restrict__ tiles, int nt, int mtk, int ncg,
                                             const int* __restrict__ eids,
-                                            const int* __restrict__ eids1) {
+                                            const int* __restrict__ eids1, bool far) {
   const int nx = gridDim.x % NXCD == 0 ? NXCD : 1;
   const int x = (int)blockIdx.x % nx, j = (int)blockIdx.x / nx, per = (int)gridDim.x / nx;
   Sched s;
@@ -175,6 +184,7 @@ __device__ __forceinline__ Sched make_sched(unsigned char* scratch, unsigned cha
     return (int)((long long)(2 * p + c) * nx / (2LL * total)) == x;
   };
   // this XCD's others, from the back of the order; its shared tiles' number and cost
+  const int na = nalone > x ? (nalone - x + nx - 1) / nx : 0;
   int ns = 0, cs = 0, ca = 0;
   for (int c = w; c < nch; c += NWAVE) {
     const int i = c * WAVE + lane;
@@ -184,7 +194,7 @@ __device__ __forceinline__ Sched make_sched(unsigned char* scratch, unsigned cha
     const int p = cost[c] + wave_incl_scan(tc) - tc;
     const int q = alone[c] + mbcnt(__ballot(oth));
     if (oth && q % nx == x) {
-      o[ORD_MAX - 1 - q / nx] = (uint16_t)i;
+      o[ORD_MAX - 1 - (TWO && far ? na - 1 - q / nx : q / nx)] = (uint16_t)i;
       ca += tile_cost(k);
     }
     if (shd && mine(p, tc)) {
@@ -201,7 +211,7 @@ __device__ __forceinline__ Sched make_sched(unsigned char* scratch, unsigned cha
     atomicAdd(&sum[4], ca);
   }
   __syncthreads();
-  const int nshared = uniform(sum[2]), na = nalone > x ? (nalone - x + nx - 1) / nx : 0;
+  const int nshared = uniform(sum[2]);
   cs = uniform(sum[3]);
   ca = uniform(sum[4]);
   if (w == 0) {                                     // its shared tiles, in list order

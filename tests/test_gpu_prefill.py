@@ -195,3 +195,41 @@ def test_layer_prefill_gemm_shapes_and_return_codes(pkg, ops):
     assert call(20, 2560, 1536, z, z) == -1 and call(20, 384, 1536, z, z) == -6
     assert call(20, 768, 2560, z, P(1)) == -6 and call(20, 2560, 1500, z, z) == -2
     assert call(0, 2560, 1536, z, z) == 0
+
+
+@pytest.mark.parametrize("K,N", [(768, 512), (1024, 512), (2560, 256)])
+def test_second_set_in_host_memory(ops, K, N):
+    """The second align's weights in pinned host memory (unshared tiles are then walked from the
+    end): the bits of the same call over device copies, eager and in a replayed graph."""
+    gen = torch.Generator(DEV).manual_seed(K + N)
+    # unshared tiles of both sets, 0 to 4 of them per XCD, beside shared ones
+    rows = [300, 40, 17, 128, 1, 0, 700, 96, 33] * 4 + [50] * 3
+    rows1 = [r if i % 2 else 0 for i, r in enumerate(rows)]
+    rows2 = [r - q for r, q in zip(rows, rows1)]
+    mtk = sum(rows)
+    order = torch.randperm(mtk, generator=torch.Generator().manual_seed(3)).tolist()
+    w0, s0 = weights(len(rows), N, K, gen)
+    w1, s1 = weights(len(rows), N, K, gen)
+    al0 = align(rows1, order[:sum(rows1)], mtk)
+    al1 = align(rows2, order[sum(rows1):], mtk)
+    host = [torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t) for t in (w1, s1)]
+    qx = torch.randint(0, 0x7f, (mtk, K), dtype=torch.uint8, generator=gen,
+                       device=DEV).view(torch.float8_e4m3fn)
+    xs = torch.rand(mtk, K // 128, generator=gen, device=DEV)
+    tw = torch.rand(mtk, generator=gen, device=DEV)
+    tiles = ops.moe_gemm_tiles_split(al0[1:], al1[1:])
+    want, y = (torch.full((mtk, N), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    gpu_case(f"prefill gemm, second set in host memory, K={K} N={N}")
+    ops.moe_gemm_prefill(want, qx, xs, w0, s0, al0, (w1, s1, al1), tw, mtk, 1, tiles)
+    call = lambda: ops.moe_gemm_prefill(y, qx, xs, w0, s0, al0, (*host, al1), tw, mtk, 1, tiles)
+    call()
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for _ in range(3):
+        y.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16))
