@@ -208,12 +208,39 @@ def moe_gemm_split_qin(y: torch.Tensor, act: torch.Tensor, w_hot: torch.Tensor,
     check(rc, "rlu_moe_gemm_split_qin")
 
 
+def _head_rows16(m: int, N: int, K: int) -> bool:
+    """Whether m rows of the fp8 head run the 16-row kernel where the 64-row one reads the weights no
+    less often: up to 8 rows, by the times below (16-row / 64-row kernel). Both split K over 4, 2 or
+    1 waves of `steps` 128-deep steps.
+    * A 64-row workgroup takes 64 columns of all 4 waves, so a short N fills too few of the 256 CUs:
+      from 4 steps on at up to 160 workgroups (N = 8192, 4 rows, K = 2048 / 2560 / 3840: 5.7 / 6.5,
+      5.8 / 7.2 and 9.3 / 13.4 us; at 192 workgroups, N = 12288, K = 2560: 7.8 / 7.7), unless the
+      16-row kernel's ring of 5 steps pads more than half of them (K = 3072, N = 1024: 5.3 / 4.5).
+    * From K = 4096 on the 16-row kernel streams better (N = 151936, 4 rows, K = 4096 / 5120 / 7168 /
+      8192: 97 / 107, 112 / 118, 156 / 163 and 214 / 225 us; at multiples of 4096 the other one's
+      strips lie a power of two apart) unless its ring pads a quarter of the steps or more
+      (K = 5632, 4 rows: 134 / 125; 6144, 4 / 8 rows: 142 / 139 and 150 / 140).
+    * One row whose steps fill that ring (K = 2560, N = 151936, 1 / 2 / 4 rows: 56 / 59, 57 / 57 and
+      61 / 58 us: it takes the rows from the L2 twice as often)."""
+    groups = K // GROUP
+    split = 4 if groups % 4 == 0 else 2 if groups % 2 == 0 else 1
+    steps = groups // split
+    if m > 8 or steps < 4:
+        return False
+    pad = -steps % 5
+    if N * split <= 160 * 256:
+        return 2 * pad <= steps
+    if K >= 4096:
+        return K % 4096 == 0 or 4 * pad < steps
+    return m == 1 and K >= 2560 and pad == 0
+
+
 def gemm_fp8_block_q(qx: torch.Tensor, xs: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor,
                      out: torch.Tensor | None = None, wv: int = 0, npw: int = 0) -> torch.Tensor:
     """e4m3 [M, K] (xs [M, K/128]) x e4m3 [N, K] in fragment order (ws [N/128, K/128])^T ->
     bf16 [M, N], one launch per 64 rows. A given wv or npw (workgroups per CU, 16-column tiles
-    per item) runs the 16-row kernel in launches of 16 rows; so do up to 8 rows of K >= 4096,
-    where it is no slower (vocab 128256 x 4096: 92 against 94 us; at K = 3584 85 against 69)."""
+    per item) runs the 16-row kernel in launches of 16 rows; so do up to 8 rows where it is the
+    faster one (_head_rows16). The same bits either way."""
     M, K = qx.shape
     N = wq.shape[0]
     assert qx.is_contiguous() and xs.is_contiguous() and xs.shape == (M, K // GROUP)
@@ -225,7 +252,7 @@ def gemm_fp8_block_q(qx: torch.Tensor, xs: torch.Tensor, wq: torch.Tensor, ws: t
         m = min(M - r0, 16 if small else 64)
         a = (_P(qx[r0].data_ptr()), _P(xs[r0].data_ptr()), _p(wq), _p(ws), _P(y[r0].data_ptr()),
              m, N, K)
-        if small or (m <= 8 and K >= 4096):
+        if small or _head_rows16(m, N, K):
             p = npw if npw else (2 if m <= 8 else 4)
             check(lib().rlu_gemm_fp8blk_m16(*a, wv, p, _P(stream_ptr())), "rlu_gemm_fp8blk_m16")
         else:

@@ -40,6 +40,27 @@ def test_fp8_head_rows_equal_16_row_launches(ops, M, K):
         assert torch.equal(y.view(torch.int16), want.view(torch.int16))
 
 
+# the 64-row kernel by itself, also where the entry point above takes the 16-row one; K / 128 = 20, 32,
+# 23, 46 and 96: 5, 8, 23, 23 and 24 steps a wave (24 the longest) of 4, 4, 1, 2 and 4 waves
+@pytest.mark.parametrize("K", [2560, 4096, 2944, 5888, 12288])
+@pytest.mark.parametrize("M", [1, 5, 8, 16, 17, 40, 64])
+def test_fp8_head_m64_equals_16_row_kernel(pkg, ops, M, K):
+    N = 1152
+    gen = torch.Generator(DEV).manual_seed(M + K)
+    w = torch.randint(0, 256, (N, K), dtype=torch.uint8, generator=gen, device=DEV)
+    w = torch.where((w & 0x7f) == 0x7f, w ^ 1, w).view(torch.float8_e4m3fn)
+    ws = torch.rand(N // 128, K // 128, generator=gen, device=DEV) * 0.01
+    qx, xs = ops.fp8_quant_group(torch.randn(M, K, generator=gen, device=DEV).bfloat16(), 128)
+    gpu_case(f"fp8 head, 64-row kernel alone, M={M} N={N} K={K}")
+    y = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    rc = pkg.lib().rlu_gemm_fp8blk_m64(*[P(t.data_ptr()) for t in (qx, xs, w, ws, y)], M, N, K,
+                                       P(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    want = ops.gemm_fp8_block_q(qx, xs, w, ws, npw=2 if M <= 8 else 4)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
 def test_fp8_head_m64_return_codes(pkg):
     f = pkg.lib().rlu_gemm_fp8blk_m64
     z, s = P(0), P(torch.cuda.current_stream().cuda_stream)
