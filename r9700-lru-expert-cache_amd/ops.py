@@ -210,29 +210,36 @@ def moe_gemm_split_qin(y: torch.Tensor, act: torch.Tensor, w_hot: torch.Tensor,
 
 def _head_rows16(m: int, N: int, K: int) -> bool:
     """Whether m rows of the fp8 head run the 16-row kernel where the 64-row one reads the weights no
-    less often: up to 8 rows, by the times below (16-row / 64-row kernel). Both split K over 4, 2 or
-    1 waves of `steps` 128-deep steps.
-    * A 64-row workgroup takes 64 columns of all 4 waves, so a short N fills too few of the 256 CUs:
-      from 4 steps on at up to 160 workgroups (N = 8192, 4 rows, K = 2048 / 2560 / 3840: 5.7 / 6.5,
-      5.8 / 7.2 and 9.3 / 13.4 us; at 192 workgroups, N = 12288, K = 2560: 7.8 / 7.7), unless the
-      16-row kernel's ring of 5 steps pads more than half of them (K = 3072, N = 1024: 5.3 / 4.5).
-    * From K = 4096 on the 16-row kernel streams better (N = 151936, 4 rows, K = 4096 / 5120 / 7168 /
-      8192: 97 / 107, 112 / 118, 156 / 163 and 214 / 225 us; at multiples of 4096 the other one's
-      strips lie a power of two apart) unless its ring pads a quarter of the steps or more
-      (K = 5632, 4 rows: 134 / 125; 6144, 4 / 8 rows: 142 / 139 and 150 / 140).
-    * One row whose steps fill that ring (K = 2560, N = 151936, 1 / 2 / 4 rows: 56 / 59, 57 / 57 and
-      61 / 58 us: it takes the rows from the L2 twice as often)."""
+    less often: up to 8 rows, by the times below (16-row / 64-row kernel, µs at 4 rows if not said,
+    weights from HBM). Both split K over 4, 2 or 1 waves of `steps` 128-deep steps; below 4 steps
+    the 64-row kernel is always the faster one. Its workgroup takes 64 columns of all 4 waves, the
+    16-row kernel's half of that, and `wgs` counts its workgroups:
+    * Up to 128 the 16-row kernel still has one round of the 256 CUs, on twice as many of them
+      (K = 2560, N = 8192: 6.3 / 7.2; K = 3840, N = 16384: 12.8 / 14.9; K = 1664, N = 32000: 11.3 /
+      13.6), unless its ring of 5 steps pads more than half of them (K = 3072, N = 8192: 7.8 /
+      7.6).
+    * From there to 256 it has a second round, nearly empty, and the 64-row kernel one (N = 10240,
+      K = 2560 / 3584 / 7168: 8.2 / 7.4, 11.5 / 9.1 and 17.3 / 14.9).
+    * Beyond, unless its ring pads a quarter of the steps or more, the 16-row kernel streams better
+      with K over 4 waves from K = 4096 on (N = 151936, K = 4096 / 5120 / 7168: 97 / 106, 113 / 120
+      and 158 / 166; over 2 waves, K = 4352: 102 / 97), at multiples of 4096, where the 64-row
+      kernel's strips lie a power of two apart, with any padding. Else it does where the 64-row
+      kernel, two workgroups to a CU, has a few CUs with a second one (K = 2560, N = 20480: 12.0 /
+      12.7) or a last round under 0.6 full (K = 3840, N = 102400: 61.6 / 65.0; K = 2944, N =
+      151936: 67.9 / 73.6; a full one, N = 128256: 57.3 / 56.8), and for one row of which 4 waves'
+      steps fill the ring (K = 2560, N = 151936, 1 / 2 / 4 rows: 56 / 59, 57 / 57 and 61 / 58)."""
     groups = K // GROUP
     split = 4 if groups % 4 == 0 else 2 if groups % 2 == 0 else 1
     steps = groups // split
     if m > 8 or steps < 4:
         return False
-    pad = -steps % 5
-    if N * split <= 160 * 256:
+    pad, wgs = -steps % 5, N * split // 256
+    if wgs <= 128:
         return 2 * pad <= steps
-    if K >= 4096:
-        return K % 4096 == 0 or 4 * pad < steps
-    return m == 1 and K >= 2560 and pad == 0
+    if wgs < 256 or (4 * pad >= steps and K % 4096):
+        return False
+    return ((K >= 4096 and split == 4) or wgs <= 352 or 512 < wgs <= 820 or
+            (m == 1 and split == 4 and pad == 0))
 
 
 def gemm_fp8_block_q(qx: torch.Tensor, xs: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor,

@@ -37,17 +37,23 @@ def fp8_route(pkg, monkeypatch):
     return route
 
 
-# the 16-row kernel where the 64-row one is slower: few workgroups, long K, one row that fills its ring
+# the 16-row kernel where the 64-row one is slower: up to 128 workgroups of it (K split over 4, 2 and 1
+# waves), long K, few CUs with a second workgroup, a last round under 0.6 full, one row that fills
+# its ring
 @pytest.mark.parametrize("M,N,K", [
-    (1, 8192, 2560), (8, 8192, 2048), (8, 10240, 2560), (8, 20480, 3840), (8, 32000, 1664),
-    (1, 151936, 2560), (4, 151936, 4096), (8, 32000, 5120), (1, 128256, 7168), (8, 151936, 8192)])
+    (1, 8192, 2560), (8, 8192, 2048), (8, 16384, 3840), (8, 32000, 1664), (2, 20480, 2560),
+    (8, 102400, 3840), (8, 151936, 2944), (1, 151936, 2560), (4, 151936, 4096), (8, 32000, 5120),
+    (1, 128256, 7168), (8, 151936, 8192), (8, 16384, 8192)])
 def test_fp8_head_16_row_kernel(fp8_route, M, N, K):
     assert fp8_route(M, N, K) == [("m16", M)]
 
 
+# (from 129 to 255 workgroups, and where the ring pads too much of the steps or they are under 4)
 @pytest.mark.parametrize("M,N,K", [
-    (2, 151936, 2560), (8, 12288, 2560), (8, 8192, 1536), (8, 8192, 3072), (8, 50304, 1664), (1, 151936, 3584),
-    (8, 151936, 6144), (4, 102400, 5632), (9, 8192, 2560), (16, 151936, 4096), (64, 4096, 4096)])
+    (2, 151936, 2560), (8, 8320, 2560), (1, 10240, 2560), (8, 12288, 8192), (8, 16256, 5120),
+    (4, 16512, 3840), (8, 50304, 1664), (8, 128256, 2944), (8, 8192, 1536), (8, 8192, 3072),
+    (1, 151936, 3584), (8, 151936, 6144), (4, 102400, 5632), (8, 50304, 5888), (9, 8192, 2560), (16, 151936, 4096),
+    (64, 4096, 4096)])
 def test_fp8_head_64_row_kernel(fp8_route, M, N, K):
     assert fp8_route(M, N, K) == [("m64", M)]
 
