@@ -134,6 +134,17 @@ def unpack_w4(packed: PackedW4, dtype: torch.dtype = torch.float32) -> torch.Ten
     return w.reshape(packed.n_pad, packed.k)[:packed.n].to(dtype)
 
 
+def _rows16(m: int, n_pad: int, k: int) -> bool:
+    """Whether m > 16 rows run the 16-row kernel all the same: up to 32 of them over few output rows,
+    where a wave of the 64-row kernel has one strip and walks all of K in a ring of 8 groups (of
+    128), which half a ring at K's end pads, and the 16-row kernel splits K over 4 waves (µs, one
+    read / launches of 16 rows, 24 rows: K = 2560, N = 1024 / 4096 / 8192: 16.7 / 15.2, 16.9 / 16.4
+    and 17.0 / 17.0; K = 3584: 21.9 / 19.6, 22.1 / 20.9 and 22.3 / 21.5). Up to K = 1024 the launches
+    count for more (N = 1024, K = 512: 6.4 / 8.1), and without the padding so does the second read
+    (K = 2048: 12.2 / 12.7, 12.4 / 13.6)."""
+    return m <= 2 * MAX_M and n_pad <= 4096 and k > 1024 and k // GROUP % 8 == 4
+
+
 def _gemm_into(x: torch.Tensor, packed_wq: torch.Tensor, packed_sz: torch.Tensor, k: int,
                y: torch.Tensor, wv: int) -> None:
     m = x.shape[0]
@@ -142,8 +153,8 @@ def _gemm_into(x: torch.Tensor, packed_wq: torch.Tensor, packed_sz: torch.Tensor
     while r0 < m:
         # up to 64 rows share one read of the weight; a rest of at most 16, or a given wv, runs the
         # 16-row kernel (16 rows at vocab 151936 x 2560: 42-46 us on either, 32000 x 4096: 23 and
-        # 24, 4096 x 2560: 13 and 17; 17 rows: 85 and 49, 42 and 29, 20 and 20)
-        many = m - r0 > MAX_M and not wv
+        # 24, 4096 x 2560: 13 and 17; 17 rows: 85 and 49, 42 and 29, 16 and 16)
+        many = m - r0 > MAX_M and not wv and not _rows16(m - r0, n_pad, k)
         r1 = min(m, r0 + (4 * MAX_M if many else MAX_M))
         a = (_P(x[r0:r1].data_ptr()), r1 - r0, k, _P(packed_wq.data_ptr()),
              _P(packed_sz.data_ptr()), _P(y[r0:r1].data_ptr()), n_pad)

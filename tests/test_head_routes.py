@@ -62,3 +62,29 @@ def test_fp8_head_row_blocks_and_given_launch_shapes(fp8_route):
     assert fp8_route(133, 32000, 4096) == [("m64", 64), ("m64", 64), ("m16", 5)]
     assert fp8_route(20, 32000, 2560, npw=4) == [("m16", 16), ("m16", 4)]
     assert fp8_route(20, 32000, 2560, wv=2) == [("m16", 16), ("m16", 4)]
+
+
+@pytest.fixture
+def w4_route(pkg, monkeypatch):
+    w4 = import_module(pkg.__name__ + ".w4")
+
+    def route(M, N, K, wv=0):
+        lib = Calls(1)
+        monkeypatch.setattr(w4, "lib", lambda: lib)
+        monkeypatch.setattr(w4, "stream_ptr", lambda: 0)
+        wq = torch.empty(1, dtype=torch.uint8).expand(N // 16, K // 128, 64, 16)
+        w4._gemm_into(torch.empty(M, K, dtype=torch.bfloat16), wq, torch.empty(1), K,
+                      torch.empty(M, N, dtype=torch.bfloat16), wv)
+        return lib.made
+    return route
+
+
+# few output rows and a K whose last half ring is padding: 16 rows at a time up to 32 of them
+@pytest.mark.parametrize("M,N,K,made", [
+    (32, 4096, 2560, [16, 16]), (17, 1024, 3584, [16, 1]), (24, 4096, 1536, [16, 8]),
+    (16, 151936, 2560, [16]), (88, 4096, 2560, [64, 16, 8]), (33, 4096, 2560, [33]),
+    (32, 4128, 2560, [32]), (32, 4096, 2048, [32]), (32, 1024, 512, [32]),
+    (17, 1024, 1792, [17]), (64, 151936, 2560, [64]), (82, 151936, 2560, [64, 18])])
+def test_w4_head_routes(w4_route, M, N, K, made):
+    assert w4_route(M, N, K) == [("m64" if m > 16 else "m16", m) for m in made]
+    assert w4_route(20, 151936, 2560, wv=2) == [("m16", 16), ("m16", 4)]
