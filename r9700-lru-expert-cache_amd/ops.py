@@ -518,7 +518,11 @@ def moe_gemm_prefill(out, qx: torch.Tensor, x_scale: torch.Tensor, w0: torch.Ten
     else:
         assert q2.shape == (mtk, N // 2) and q2.dtype == FP8 and q2.is_contiguous()
         assert s2.shape == (mtk, N // 256) and s2.dtype == torch.float32 and s2.is_contiguous()
-    assert qx.dtype == FP8 and w0.dtype == FP8 and qx.shape[1] == K
+    assert qx.dtype == FP8 and w0.dtype == FP8 and qx.shape[1] == K and qx.is_contiguous()
+    # the kernel reads these by row number alone, up to row (mtk - 1) // top_k
+    assert qx.shape[0] * top_k >= mtk
+    for t, n in ((x_scale, qx.shape[0] * (K // GROUP)), (topk_weights, mtk)):
+        assert t is None or (t.dtype == torch.float32 and t.is_contiguous() and t.numel() >= n)
     nb = al0[1].numel()
     b = [_P(0)] * 4
     if second is not None:
