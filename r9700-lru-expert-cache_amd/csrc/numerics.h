@@ -75,10 +75,11 @@ __device__ __forceinline__ float silu_bf16(float g) {
 
 // silu_bf16 of a bf16 value with the chip's exponential and reciprocal (v_exp_f32, v_rcp_f32): with z
 // = e^-|g|, (g < 0 ? g z : g) / (1 + z). The reduction leaves v_exp_f32 an argument in [-0.5, 0.5],
-// 1 + z is in [1, 2] and its reciprocal refined once, so s is within a few float32 ulps of the
-// quotient above and rounds to the same bf16 for every one of the 2^16 inputs, NaN, infinities
-// and denormals included; the library's self-test rlu_selftest_silu checks all of them on the
-// device. The prefill SiLU-mul-quant epilogue and silu_mul_quant spend their time on such vector
+// 1 + z is in [1, 2] and its reciprocal refined once. That bounds s less tightly than its bf16 needs: the
+// reduction's float32 log2(e) is 1.3e-8 too small, which in z is |g| times that, 2 float32 ulps at
+// g = -16 and 10 at -88, beside the two instructions' own errors. That s rounds to the same bf16 as
+// the quotient above for every one of the 2^16 inputs, NaN, infinities and denormals included, is
+// what the library's self-test rlu_selftest_silu finds on the device, trying them all. The prefill SiLU-mul-quant epilogue and silu_mul_quant spend their time on such vector
 // instructions, and this has under half of silu_bf16's: gate_up with its activation at 8192 tokens
 // over 512 experts 715 -> 685 us, over 128 experts of hidden 2048 431 -> 405 us, silu_mul_quant of
 // 81920 x 768 113 -> 90 us.

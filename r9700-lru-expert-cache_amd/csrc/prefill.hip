@@ -14,10 +14,11 @@
 //   * An item is (tile of <= 8 16-row blocks of one expert, 16 S W output columns). Each of the
 //     W waves owns S 16-column weight strips and computes every block of the tile for them, so
 //     a weight fragment is used from registers by all the tile's blocks and never goes through
-//     LDS. Each wave streams its strips through a ring of D register stages (global loads,
-//     nontemporal) with no barrier on them, and the ring runs on across item boundaries: the
-//     last D steps of an item issue the first D steps of the next one. ~160 KB of weights are
-//     in flight per CU.
+//     LDS. Each wave streams its strips through a ring of D register stages (buffer loads,
+//     streaming, or with the plain cache policy where an expert has several tiles) with no
+//     barrier on them, and the ring runs on across item boundaries: the last D steps of an item
+//     issue the first D steps of the next one. Up to D x 32 KB = 192 KB of weights are in flight
+//     per CU.
 //   * The tile's activation rows (gathered through sorted_ids) go to LDS in chunks of KC K
 //     steps, double-buffered, loaded into registers one whole chunk ahead -- the next item's
 //     first chunk during this item's last one -- and written at the chunk's end, so waiting

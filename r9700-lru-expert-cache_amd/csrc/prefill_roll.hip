@@ -7,8 +7,11 @@
 // two kinds differ less (64 tokens: 68 against 79 us, and 37 against 39).
 //
 // Bound: with few rows per tile the weight read (all 512 experts of gate_up, 2.01 GB, in 330-345
-// us = 5.9-6.1 TB/s; a bare read in this pattern, 7.0); with full tiles the chip's power (the
-// clock drops to 1.8-2.1 GHz) and the LDS, at 1.2-1.3 PFLOP/s with the weights in the L2.
+// us = 5.9-6.1 TB/s; a bare read in this pattern, 7.0); with full tiles, at 1.2-1.3 PFLOP/s with the
+// weights in the L2, three units that overlap only in part: a step of 8 blocks is 32 cycles for each of
+// a SIMD's 32 MFMAs, 128 KB of LDS reads (each fragment feeds two MFMAs), about as long, and the
+// scaling of every product. Counted over 32 experts' full tiles with the activation: MFMA busy
+// 23% of the cycles, LDS 21% (1% conflicts), vector instructions 40%, at 2.2 GHz.
 //
 //   * An item is (tile of <= 8 16-row blocks of one expert, 256 columns); wave w of 8 owns 2
 //     16-column weight strips and streams them through a ring of KC = 4 register steps that runs
