@@ -444,10 +444,9 @@ def prefill_gemm(torch, pkg, dev, T=4096, reps=3, lru=True, wv=0):
     sq2 = torch.empty(mtk, I // 128, dtype=torch.float32, device=dev)
     u_act = timed(lambda: ops.silu_mul_quant(y1, out=(q2, sq2)))
     u_fused = None
-    if wv == 0 and ops.moe_gemm_tiled_silu_quant_built(H, 2 * I):
-        u_fused = timed(lambda: ops.moe_gemm_tiled_silu_quant(q2, sq2, x, xs, w13, w13s, sh, eh,
-                                                              nh, mtk, TOPK, tiles=tiles,
-                                                              tiles_ready=True))
+    if wv == 0 and ops.moe_gemm_prefill_takes(mtk, H, 2 * I, act=True):
+        u_fused = timed(lambda: ops.moe_gemm_prefill((q2, sq2), x, xs, w13, w13s, (sh, eh, nh),
+                                                     None, None, mtk, TOPK, tiles))
     # the fused LRU + both aligns (+ the group-128 quant of the chunk's hidden states, as the
     # layer calls it) over the chunk's 40960 (token, k) ids
     ids_d = torch.from_numpy(ids).to(dev).reshape(-1)

@@ -244,9 +244,9 @@ int rlu_moe_gemm_fp8blk_tiled_silu_quant(const void* qx, const float* xs, const 
  *     each (-1 otherwise, or on a NULL pointer).
  *   rlu_moe_gemm_fp8blk_tiled_split / _split_silu_quant: rlu_moe_gemm_fp8blk_tiled (wv = 0) /
  *     rlu_moe_gemm_fp8blk_tiled_silu_quant on each align, in one launch, equal to the two calls
- *     bit for bit; max_tiles = nb_max0 + nb_max1. Built for the streamed kernel's shapes (K =
- *     2560 or 768 and N % 256 == 0; K = 2560 for _silu_quant): other shapes return -6 before
- *     any other check, so a call with mtk = 0 is a capability query. Every pointer but
+ *     bit for bit; max_tiles = nb_max0 + nb_max1. Taken: K = 2560 or 768 and N % 256 == 0 (K =
+ *     2560 for _silu_quant); other shapes return -6 before any other check, also those that
+ *     rlu_moe_gemm_prefill takes, so a call with mtk = 0 is a capability query. Every pointer but
  *     topk_weights is required (-1); otherwise -1 / -2 as rlu_moe_gemm_fp8blk_tiled. */
 int rlu_moe_gemm_tiles_split(const int* expert_ids0, const int* num_post_pad0, int nb_max0,
                              const int* expert_ids1, const int* num_post_pad1, int nb_max1,

@@ -14,7 +14,8 @@ struct PfSecond {
   const int* expert_ids;
 };
 
-// K and N of the two-set entry points.
+// K and N of the two-set entry points of gemm_tiled.hip (rlu_moe_gemm_prefill's are
+// prefill_stream_takes).
 bool prefill_stream_built(int K, int N);
 
 // Whether the launches below take mtk rows of this shape (act: the one with the activation).
@@ -31,7 +32,7 @@ int launch_prefill_stream(const void* qx, const float* xs, const void* wq, const
 
 // The same kernel for gate_up with SiLU-mul-quant in its epilogue: writes q2 [mtk, N / 2] e4m3
 // and s2 [mtk, N / 256] (group-128 scales) instead of the bf16 output. Returns -1 (nothing
-// launched) where roll_takes says no; prefill_stream_act_built: the shapes of its entry points.
+// launched) where roll_takes says no; prefill_stream_act_built: the K and N of the _silu_quant entry points.
 bool prefill_stream_act_built(int K, int N);
 int launch_prefill_stream_act(const void* qx, const float* xs, const void* wq, const float* ws,
                               const int* sorted_ids, const int* expert_ids,

@@ -389,8 +389,8 @@ def moe_gemm_tiled(y: torch.Tensor, qx: torch.Tensor, x_scale: torch.Tensor, wq:
 
 
 def moe_gemm_tiled_silu_quant_built(K: int, N: int) -> bool:
-    """Whether moe_gemm_tiled_silu_quant has a kernel for gate_up weights [*, N, K] (a
-    zero-row call: nothing is launched)."""
+    """Whether moe_gemm_tiled_silu_quant takes gate_up weights [*, N, K] (a zero-row call: nothing
+    is launched); moe_gemm_prefill, the layer's call, takes more shapes."""
     rc = lib().rlu_moe_gemm_fp8blk_tiled_silu_quant(
         *([_P(0)] * 8), 1, _P(0), _P(0), 0, 1, K, N, _P(0))
     return rc == 0
@@ -445,8 +445,8 @@ def _split_tiles(al0, al1, tiles, ready):
 
 
 def moe_gemm_tiled_split_built(K: int, N: int) -> bool:
-    """Whether moe_gemm_tiled_split has a kernel for weights [*, N, K] (a zero-row call:
-    nothing is launched)."""
+    """Whether moe_gemm_tiled_split takes weights [*, N, K] (a zero-row call: nothing is launched);
+    moe_gemm_prefill, the layer's call, takes more shapes."""
     rc = lib().rlu_moe_gemm_fp8blk_tiled_split(*([_P(0)] * 12), 1, _P(0), _P(0), 0, 1, K, N,
                                                _P(0))
     return rc == 0
