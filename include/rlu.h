@@ -381,6 +381,10 @@ int rlu_selftest_silu(unsigned long long* bad, hipStream_t stream);
  * 0, -1 (bad sizes or NULL), -2 (K % 128, K < 512, or rows * K past 2 GB). */
 int rlu_selftest_prefill_rows(int rows, int K, unsigned long long* bad);
 
+/* Likewise: the weight steps of K (128 deep) that a workgroup of that kernel loads for `items` items.
+ * Returns 0, -1 (bad sizes or NULL), -2 (K % 128 or K < 512). */
+int rlu_selftest_prefill_steps(int items, int K, unsigned long long* steps);
+
 #ifdef __cplusplus
 }
 #endif

@@ -55,6 +55,7 @@ SIGNATURES: dict[str, tuple] = {
     "rlu_selftest_bf16": (_I, [_P, _P]),
     "rlu_selftest_silu": (_I, [_P, _P]),
     "rlu_selftest_prefill_rows": (_I, [_I, _I, _P]),
+    "rlu_selftest_prefill_steps": (_I, [_I, _I, _P]),
 }
 
 

@@ -93,6 +93,16 @@ __host__ __device__ __forceinline__ void row_loads(int qbytes, int nk, int va, i
   }
 }
 
+// The weight steps that chunk c's walk loads ahead: the next chunk's, of this item or (last) of the next.
+// After a workgroup's last item (!more) none: its first KC steps again would be 33 MB over 256
+// workgroups, 0.55 ms where the weights come over the host link (gate_up over 256 experts, half of
+// them in host memory, 195 tokens: layer step 4.68 -> 4.09 ms).
+template <bool TAIL>
+__host__ __device__ __forceinline__ int steps_ahead(int nk, int c, bool last, bool more) {
+  if (last) return more ? KC : 0;
+  return TAIL ? nk - (c + 1) * KC : KC;
+}
+
 // ACT: SiLU-mul-quant in the epilogue. N = 2 I (gate | up); item g covers gate columns [128 g,
 // 128 g + 128) (waves 0 .. 3) and the matching up columns [I + 128 g, ...) (waves 4 .. 7), so
 // each output row's 128-column activation group is whole in one item. The epilogue writes q2
@@ -305,7 +315,7 @@ __device__ __forceinline__ void items(
       const bool last = c + 1 == nch;
       const uint8_t* bld = last ? bnext : bcur;
       const int woff = last ? 0 : (c + 1) * KC * 2048;
-      const int ahead = TAIL && !last ? nk - (c + 1) * KC : KC;   // steps of the next chunk
+      const int ahead = steps_ahead<TAIL>(nk, c, last, m + 1 < cnt);   // steps of the next chunk
       const int here = TAIL && last ? nk - c * KC : KC;           // ... of this one
       // the next chunk: this item's, or the next item's first
       Rows st = rA;
@@ -366,7 +376,7 @@ __device__ __forceinline__ void items(
 #pragma unroll
       for (int ks = 0; ks < KC; ++ks) {
         if (TAIL && ks >= here) {                   // (uniform) the ring runs on
-          issue_b(ks, wbuf(bld, ks < ahead), woff + ks * 2048);
+          issue_b(ks, wbuf(bld, TAIL ? ks < ahead : ahead > 0), woff + ks * 2048);
           continue;
         }
         if (r6) {
@@ -389,7 +399,7 @@ __device__ __forceinline__ void items(
         }
         unit(ks, 1, true);
         unit(ks, 0, false);
-        issue_b(ks, wbuf(bld, ks < ahead), woff + ks * 2048);
+        issue_b(ks, wbuf(bld, TAIL ? ks < ahead : ahead > 0), woff + ks * 2048);
         scale(0);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -544,6 +554,16 @@ static int loads_outside(int rows, int K) {
   return bad;
 }
 
+// the weight steps a workgroup of `items` items loads, the ring's first fill and what follows
+template <bool TAIL>
+static long long steps_loaded(int items, int nk) {
+  long long steps = KC;
+  for (int m = 0; m < items; ++m)
+    for (int c = 0; c < chunks<TAIL>(nk); ++c)
+      steps += max(0, min(KC, steps_ahead<TAIL>(nk, c, c + 1 == chunks<TAIL>(nk), m + 1 < items)));
+  return steps;
+}
+
 }  // namespace roll
 
 void launch_roll(const Args& a, int max_tiles, hipStream_t stream) {
@@ -600,5 +620,15 @@ extern "C" int rlu_selftest_prefill_rows(int rows, int K, unsigned long long* ba
   if (rows < 1 || K < 1 || !bad) return -1;
   if (K % 128 || K < 512 || (long long)rows * K > 0x7fffffff) return -2;
   *bad = has_tail(K) ? loads_outside<true>(rows, K) : loads_outside<false>(rows, K);
+  return 0;
+}
+
+// Host only: the weight steps (of 128 deep, 32 KB) that a workgroup of the rolled kernel loads for `items`
+// items of K. Returns -1 (bad sizes or NULL), -2 (K % 128 or K < 512).
+extern "C" int rlu_selftest_prefill_steps(int items, int K, unsigned long long* steps) {
+  using namespace rlu::pf::roll;
+  if (items < 1 || K < 1 || !steps) return -1;
+  if (K % 128 || K < 512) return -2;
+  *steps = has_tail(K) ? steps_loaded<true>(items, K / 128) : steps_loaded<false>(items, K / 128);
   return 0;
 }
